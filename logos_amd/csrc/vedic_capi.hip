@@ -33,9 +33,9 @@ hipError_t launch_gemm_f16_direct_amp(const GemmArgs& a, hipStream_t s);
 hipError_t launch_gemm_f16_gather(const GemmArgs& a, bool amp, hipStream_t s);
 hipError_t launch_gemm_f16_skinny(const GemmArgs& a, hipStream_t s);
 hipError_t launch_gemm_f32_skinny(const GemmArgs& a, hipStream_t s);
-hipError_t launch_gemm_f32_direct_nn(const GemmArgs& a, hipStream_t s);
-hipError_t launch_gemm_f32_direct_nt(const GemmArgs& a, hipStream_t s);
-hipError_t launch_gemm_f32_direct_tn(const GemmArgs& a, hipStream_t s);
+hipError_t launch_gemm_f32_direct_nn(bool vec, const GemmArgs& a, hipStream_t s);
+hipError_t launch_gemm_f32_direct_nt(bool vec, const GemmArgs& a, hipStream_t s);
+hipError_t launch_gemm_f32_direct_tn(bool vec, const GemmArgs& a, hipStream_t s);
 }  // namespace vedic
 
 namespace vedic {
@@ -68,7 +68,6 @@ static int hip_status(hipError_t e) {
 static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Largest leading dimension (elements) the kernels' 32-bit tile offsets allow.
-static constexpr int64_t kMaxLd = int64_t(1) << 22;
 
 // Temporary device memory of library calls (split-K partial slabs, column
 // partials, the AMP cast buffer, attention partials and padded copies) comes
@@ -417,13 +416,13 @@ static hipError_t colsum_matrix(const float* X, int64_t ldx, int M, int N, float
     return e != hipSuccess ? e : f;
 }
 
-// fp32 tiles: the direct-load pipelined kernel where the operands allow
-// 16-byte loads and 32-bit tile offsets, else the element-wise kernel.
+// fp32 tiles: the split kernel (rows of any alignment) where the operands
+// allow 32-bit tile offsets, else the kernel with 64-bit element addresses.
 static hipError_t launch_f32_tiled(int op, bool vec, const GemmArgs& a, hipStream_t s) {
-    if (vec && a.lda < kMaxLd && a.ldb < kMaxLd)
-        return op == VEDIC_OP_NN   ? launch_gemm_f32_direct_nn(a, s)
-               : op == VEDIC_OP_NT ? launch_gemm_f32_direct_nt(a, s)
-                                   : launch_gemm_f32_direct_tn(a, s);
+    if (a.lda < kMaxLd && a.ldb < kMaxLd)
+        return op == VEDIC_OP_NN   ? launch_gemm_f32_direct_nn(vec, a, s)
+               : op == VEDIC_OP_NT ? launch_gemm_f32_direct_nt(vec, a, s)
+                                   : launch_gemm_f32_direct_tn(vec, a, s);
     return launch_gemm_f32(op, vec, a, s);
 }
 
@@ -433,7 +432,23 @@ static hipError_t launch_f32_tiled(int op, bool vec, const GemmArgs& a, hipStrea
 // an fp32 MFMA does an eighth of the work per cycle of an fp16 one, so a
 // slice carries the fixed prologue / epilogue cost in fewer steps).
 // 1 = no split.
+//
+// fp32 products on the split kernel (f32_use_split) with 128 x 128 tiles for
+// half the CUs or more, but not for all: slices of at least 384 steps up to
+// the three workgroups a CU holds (2048 x 1024 x 1024 NN, 128 tiles: 47.8 us
+// unsplit, 35.3 in two slices, 37.2 in four; 1001 x 1999 x 2047 TN 89.0, 60.6,
+// 60.4), within kSplitBytes of partials, so that a caller with a fixed scratch
+// region is never refused for them.
+static constexpr int64_t kSplitBytes = int64_t(24) << 20;
 static int choose_ksplit(int M, int N, int K, int cus, bool f16) {
+    const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    if (!f16 && t128 * 2 >= cus && f32_use_split(M, N, K, true, cus)) {
+        if (t128 >= cus) return 1;
+        int64_t s = 3 * (int64_t)cus / t128;
+        s = s < K / 384 ? s : K / 384;
+        s = s < kSplitBytes / (4 * (int64_t)M * N) ? s : kSplitBytes / (4 * (int64_t)M * N);
+        return s >= 2 ? (int)s : 1;
+    }
     if (f16) {
         const int64_t big = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
         if (big >= cus) return 1;  // the 256 x 256 kernel fills the GPU

@@ -94,9 +94,13 @@ enum : int {
 
 constexpr int kMaxHeads = 64;  // scatter targets per GEMM
 
-// Tile choice of the fp32 GEMM, shared by the kernel launch and the split-K
-// planner: 64 x 64 tiles when N > 64 (narrower outputs take 256 x 64 tiles)
-// and 128 x 128 tiles would cover at most half the CUs.
+// Leading dimensions below this keep a tile's row offsets in 32 bits.
+constexpr int64_t kMaxLd = int64_t(1) << 22;
+
+// Outputs with few tiles, as the fp32 kernel launches and the split-K planner
+// see them: 64 x 64 tiles when N > 64 (narrower outputs take 256 x 64 tiles,
+// 64 x 64 with unaligned rows) and 128 x 128 tiles would cover at most half
+// the CUs.
 inline bool f32_small_tiles(int M, int N, int cus) {
     return N > 64 && (int64_t)((M + 127) / 128) * ((N + 127) / 128) * 2 <= cus;
 }
@@ -111,6 +115,25 @@ inline bool f32_wave_split(int M, int N, int cus) {
     const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
     const int64_t t32 = (int64_t)((M + 31) / 32) * ((N + 63) / 64);
     return t64 < cus && t32 * 2 >= cus;
+}
+
+// Whether an fp32 product runs on the bf16 split kernel (vedic_gemm_f32s.hpp)
+// rather than on v_mfma_f32_32x32x2_f32 (vedic_gemm_f32.hpp).  The split
+// kernel's stage of 16 steps costs a CU about 0.7 us alone whatever the tile,
+// so it wants tiles for half the CUs and, where it has no more, a contraction
+// long enough to be split over workgroups: 2048 x 1024 (128 tiles of 128 x 128)
+// K = 1024 35.3 / 35.7 / 35.0 us (NN / NT / TN) against 38.4 / 35.8 / 43.3, but
+// K = 256 15.2 / 14.0 / 15.6 against 12.5 / 12.0 / 13.6; 1024 x 1024 x 1024 (64
+// tiles, four slices) 25.9 / 25.3 / 26.2 against 25.6 / 21.2 / 29.0; from 192
+// tiles up it is faster throughout (4096 x 1024 x 256 16.7 against 23.0).
+// Rows that are not 16-byte aligned, which the other kernel cannot load, always
+// run on it (512 x 1000 x 1000 with a pitch of 1001: 29.7 against 70.9 us on
+// the element-wise kernel).
+inline bool f32_use_split(int M, int N, int K, bool vec, int cus) {
+    if (!vec) return true;
+    if (N <= 64) return false;
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    return tiles * 2 > cus || (tiles * 2 == cus && K >= 512);
 }
 
 struct GemmArgs {

@@ -1,4 +1,4 @@
-// vedic_gemm_f32.hpp -- the strict-fp32 GEMM for gfx950 (v_mfma_f32_32x32x2_f32).
+// vedic_gemm_f32.hpp -- the fp32 GEMM on v_mfma_f32_32x32x2_f32 (gfx950), for small outputs.
 //
 //   C[M x N] = epi(op(A) . op(B)), A, B and C binary32, op NN / NT / TN as in
 //   the fp16 kernel (vedic_gemm_f16.hpp), whose organisation this follows:
@@ -7,11 +7,11 @@
 //   fence-free barriers, the next tile's first stages in flight during the
 //   epilogue.
 //
-// An fp32 MFMA does an eighth of the work of an fp16 one per cycle (4096
-// flops in 64 cycles), so per byte loaded there is 16x more matrix-core time:
-// the tile is 128 x 128 with four waves of 64 x 64, and the pipeline is about
-// latency, not bandwidth -- the next 32-deep stage (32 KiB) is in flight while
-// one is consumed, and a second resident workgroup covers the rest.
+// These tiles serve the products with few output tiles and those with at most
+// 64 columns (f32_use_split, vedic_common.hpp); larger ones run on the bf16
+// matrix cores (vedic_gemm_f32s.hpp).  An fp32 MFMA does an eighth of the work
+// of an fp16 one per cycle (4096 flops in 64 cycles), so per byte loaded there
+// is 16x more matrix-core time: the pipeline is about latency, not bandwidth.
 //
 // LDS layouts (32 k per stage):
 //  * KC (contraction contiguous in memory: A in NN/NT, B in NT): one 128-byte
@@ -380,18 +380,6 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f32_kernel(GemmArgs 
 #undef VEDIC_A_TILE32
 #undef VEDIC_B_TILE32
 
-// 128 x 128 tiles, four waves of 64 x 64, ST stages of 32 KiB.  Two stages
-// leave room for two workgroups per CU (2 x 64 KiB of LDS), and two
-// workgroups -- two waves per SIMD -- keep the matrix pipe busier than deeper
-// pipelines with one (measured on the 8192 x 8192 x 1024 LM head: 86 % of the
-// fp32 MFMA peak at ST = 2, 74 % at ST = 4).
-#ifndef VEDIC_F32_STAGES
-#define VEDIC_F32_STAGES 2
-#endif
-struct CfgF32 {
-    static constexpr int BM = 128, BN = 128, ST = VEDIC_F32_STAGES, WGM = 2, WGN = 2;
-    static constexpr int PER_CU = ST <= 2 ? 2 : 1;  // resident workgroups per CU (LDS: ST x 32 KiB)
-};
 // Narrow outputs (N <= 64, e.g. an attention head's P V, dQ, dK, dV at
 // DH = 64): 256 x 64 tiles, four waves of 64 x 64 stacked in M, so no MFMA
 // work lands on columns past N.  Two stages of 40 KiB, two workgroups per CU.
@@ -444,8 +432,7 @@ static hipError_t launch_f32_kind(const GemmArgs& a, hipStream_t s) {
     }
 }
 
-// Few output tiles (128 x 128 tiles for at most half the CUs, e.g. the
-// 512 x 1024 output of BASELINE config 1): 64 x 64 tiles, four waves of
+// Few output tiles (128 x 128 tiles for at most half the CUs): 64 x 64 tiles, four waves of
 // 32 x 32, four 16 KiB stages, two workgroups per CU -- four times the
 // workgroups, and deeper contraction slices once the product is split.
 struct CfgF32Small {
@@ -471,23 +458,33 @@ static_assert(CfgF32Narrow::BN == 64, "f32_small_tiles assumes the narrow tile's
 // (512 x 1024 x 1024: 12.2-13.1 us against 15.9-16.5 us on the wave-split
 // tiles).  NT keeps the wave-split tiles (its B rows are K-contiguous).
 hipError_t launch_gemm_f32_rowblocks(const GemmArgs& a, hipStream_t s);
-#ifndef VEDIC_F32_ROWBLOCKS
-#define VEDIC_F32_ROWBLOCKS 1
-#endif
 
-// Narrow tiles when N fits one 64-wide tile column; small ones when 128 x 128
-// tiles would leave most CUs idle.
+// The products f32_use_split leaves here: narrow tiles when N fits one
+// 64-wide tile column, small ones otherwise.
 template <int OP>
-hipError_t launch_gemm_f32_direct_op(const GemmArgs& a, hipStream_t s) {
+hipError_t launch_gemm_f32_mfma_op(const GemmArgs& a, hipStream_t s) {
     if (a.N <= CfgF32Narrow::BN) return launch_f32_kind<OP, CfgF32Narrow>(a, s);
     if constexpr (OP != 2) {  // (TN's A is M-contiguous: its LDS rows need at least 64 of M)
         if (a.ksplit <= 1 && f32_wave_split(a.M, a.N, device_cu_count())) {
-            if (OP == 0 && VEDIC_F32_ROWBLOCKS) return launch_gemm_f32_rowblocks(a, s);
-            return launch_f32_kind<OP, CfgF32WaveK>(a, s);
+            if constexpr (OP == 0) return launch_gemm_f32_rowblocks(a, s);
+            else return launch_f32_kind<OP, CfgF32WaveK>(a, s);
         }
     }
-    if (f32_small_tiles(a.M, a.N, device_cu_count())) return launch_f32_kind<OP, CfgF32Small>(a, s);
-    return launch_f32_kind<OP, CfgF32>(a, s);
+    return launch_f32_kind<OP, CfgF32Small>(a, s);
 }
+
+#define VEDIC_F32_KERNEL(OP, Cfg, KIND)                                                                           \
+    template __global__ void gemm_f32_kernel<OP, Cfg::BM, Cfg::BN, Cfg::ST, Cfg::WGM, Cfg::WGN, KIND,               \
+                                             WavesK<Cfg>::value>(GemmArgs)
+#define VEDIC_F32_KINDS(OP, Cfg)                  \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_PLAIN);          \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_BIAS);           \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_BIAS_GELU);      \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_BIAS_GELU_PRE);  \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_ACCUM);          \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_GENERIC);        \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_GELU_BWD);       \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_LINEAR_CS);      \
+    VEDIC_F32_KERNEL(OP, Cfg, EK_RESIDUAL)
 
 }  // namespace vedic

@@ -1,30 +1,20 @@
-// vedic_gemm_f32_nt.hip -- instantiates the strict-fp32 GEMM for op NT (one
-// translation unit per op so the build compiles them in parallel).  The kernels
-// are instantiated explicitly so that every launch has its host stub.
+// vedic_gemm_f32_nt.hip -- fp32 kernels, NT: B stored [N x K].
 #include "vedic_gemm_f32.hpp"
+#include "vedic_gemm_f32s.hpp"
 
 namespace vedic {
 
-#define VEDIC_F32_INST(KIND)                                                                                  \
-    template __global__ void gemm_f32_kernel<1, CfgF32::BM, CfgF32::BN, CfgF32::ST, CfgF32::WGM, CfgF32::WGN, KIND>(  \
-        GemmArgs);                                                                                                \
-    template __global__ void gemm_f32_kernel<1, CfgF32Narrow::BM, CfgF32Narrow::BN, CfgF32Narrow::ST,              \
-                                             CfgF32Narrow::WGM, CfgF32Narrow::WGN, KIND>(GemmArgs);                 \
-    template __global__ void gemm_f32_kernel<1, CfgF32Small::BM, CfgF32Small::BN, CfgF32Small::ST,                 \
-                                             CfgF32Small::WGM, CfgF32Small::WGN, KIND>(GemmArgs); \
-    template __global__ void gemm_f32_kernel<1, CfgF32WaveK::BM, CfgF32WaveK::BN, CfgF32WaveK::ST,                 \
-                                             CfgF32WaveK::WGM, CfgF32WaveK::WGN, KIND, CfgF32WaveK::WGK>(GemmArgs);
-VEDIC_F32_INST(EK_PLAIN)
-VEDIC_F32_INST(EK_BIAS)
-VEDIC_F32_INST(EK_BIAS_GELU)
-VEDIC_F32_INST(EK_BIAS_GELU_PRE)
-VEDIC_F32_INST(EK_ACCUM)
-VEDIC_F32_INST(EK_GENERIC)
-VEDIC_F32_INST(EK_GELU_BWD)
-VEDIC_F32_INST(EK_LINEAR_CS)
-VEDIC_F32_INST(EK_RESIDUAL)
-#undef VEDIC_F32_INST
+VEDIC_F32_KINDS(1, CfgF32Narrow);
+VEDIC_F32_KINDS(1, CfgF32Small);
+VEDIC_F32_KINDS(1, CfgF32WaveK);
+VEDIC_F32S_KINDS(1, CfgSLarge);
+VEDIC_F32S_KINDS(1, CfgSMid);
+VEDIC_F32S_KERNEL(1, false, CfgSMid, EK_GENERIC);
+VEDIC_F32S_KERNEL(1, false, CfgSSmall, EK_GENERIC);
 
-hipError_t launch_gemm_f32_direct_nt(const GemmArgs& a, hipStream_t s) { return launch_gemm_f32_direct_op<1>(a, s); }
+hipError_t launch_gemm_f32_direct_nt(bool vec, const GemmArgs& a, hipStream_t s) {
+    if (!f32_use_split(a.M, a.N, a.K, vec, device_cu_count())) return launch_gemm_f32_mfma_op<1>(a, s);
+    return vec ? launch_gemm_f32s_op<1, true>(a, s) : launch_gemm_f32s_op<1, false>(a, s);
+}
 
 }  // namespace vedic
