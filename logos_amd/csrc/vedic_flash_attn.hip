@@ -34,6 +34,7 @@
 #include <algorithm>
 
 #include "vedic_flash_device.hpp"
+#include "vedic_flash_split.hpp"
 
 namespace vedic {
 
@@ -47,32 +48,27 @@ constexpr int fa_stage_bytes() {
 #ifndef VEDIC_FA_ST128
 #define VEDIC_FA_ST128 2
 #endif
+#ifndef VEDIC_FA_WPE64
+#define VEDIC_FA_WPE64 3
+#endif
 #ifndef VEDIC_FA_WPE128
 #define VEDIC_FA_WPE128 2
 #endif
 // LDS stages in flight
 template <int DH>
 constexpr int fa_stages() {
-    return DH == 128 ? VEDIC_FA_ST128 : kFaStages;
+    return 2;
 }
 
-// One work item (`item` in decreasing size order) with the workgroup's three
-// LDS stages t0, t1, t2.
+struct FaItem {
+    int head, g, k_lo, nkb, nch;
+    int64_t asc;
+};
+
+// Work item `item` in decreasing size order.
 template <int DH>
-__device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, char* t1, char* t2) {
-    constexpr int KB = kFaKeys * DH * 4;  // bytes of one K (or V) block
-    constexpr int SB = fa_stage_bytes<DH>();
-    constexpr int NLD = SB / 1024 / 4;    // 1 KiB direct loads per wave per stage
-    constexpr int CPR = DH / 4;           // 16-byte chunks per row
-    constexpr int HALF = DH / 2;
-    static_assert(DH == 64 || DH == 128, "head dimension 64 or 128");
-    constexpr int FST = fa_stages<DH>();
-    char* const stg[3] = {t0, t1, t2};
-
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
-
-    // Work item: heads interleaved, query groups from the last (largest) down.
+__device__ __forceinline__ FaItem fa_work(const FlashArgs& a, int item) {
+    // Heads interleaved, query groups from the last (largest) down.
     const int head = item % a.nheads;
     const int64_t asc = (int64_t)a.items - 1 - item / a.nheads;
     int lo = 0, hi = a.nqg - 1;  // largest g with prefix(g) <= asc
@@ -87,6 +83,72 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
     const int kend = fa_kend(a, g);
     const int k_lo = c * a.chunk, k_hi = min(kend, k_lo + a.chunk);
     const int nkb = (k_hi - k_lo + kFaKeys - 1) / kFaKeys;
+    return {head, g, k_lo, nkb, nch, asc};
+}
+
+// An item's results: O / L and the log-sum-exp of its rows, or its slot of
+// partials.  l_run holds each lane half's sums; O is `unscale` (a power of two)
+// times the accumulators.
+template <int DH>
+__device__ __forceinline__ void fa_store(const FlashArgs& a, const FaItem& w, const float16_t (&o)[DH / 32], float m_run,
+                                         float l_run, float unscale, int wave, int lane) {
+    const int l32 = lane & 31, h = lane >> 5;
+    const int query = w.g * kFaQ + 32 * wave + l32;
+    // Row sums: each lane half summed its own 16 keys per block.
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    // o[d][4 gg + r] is O[query][32 d + 8 gg + 4 h + r].
+    if (w.nch == 1) {
+        if (query >= a.seq) return;
+        if (a.lse[w.head] != nullptr && h == 0) a.lse[w.head][query] = fa_lse(m_run, l_tot);
+        const float inv = l_tot > 1e-9f ? 1.0f / l_tot * unscale : 0.0f;
+        float* orow = a.o[w.head] + (int64_t)query * DH;
+#pragma unroll
+        for (int d = 0; d < DH / 32; ++d)
+#pragma unroll
+            for (int gg = 0; gg < 4; ++gg) {
+                float4_t v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = o[d][4 * gg + r] * inv;
+                store16_hold(orow + 32 * d + 8 * gg + 4 * h, v);
+            }
+    } else {
+        // partial slot: [kFaQ][DH] unnormalised O, then the row maxima and sums
+        float* slot = a.part + ((int64_t)w.head * a.items + w.asc) * (kFaQ * DH + 2 * kFaQ);
+        float* orow = slot + (int64_t)(32 * wave + l32) * DH;
+#pragma unroll
+        for (int d = 0; d < DH / 32; ++d)
+#pragma unroll
+            for (int gg = 0; gg < 4; ++gg) {
+                float4_t v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = o[d][4 * gg + r] * unscale;
+                store16_hold(orow + 32 * d + 8 * gg + 4 * h, v);
+            }
+        if (h == 0) {
+            slot[kFaQ * DH + 32 * wave + l32] = m_run;
+            slot[kFaQ * DH + kFaQ + 32 * wave + l32] = l_tot;
+        }
+    }
+}
+
+// One work item (`item` in decreasing size order) with the workgroup's two
+// LDS stages t0, t1.
+template <int DH>
+__device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, char* t1) {
+    constexpr int KB = kFaKeys * DH * 4;  // bytes of one K (or V) block
+    constexpr int SB = fa_stage_bytes<DH>();
+    constexpr int NLD = SB / 1024 / 4;    // 1 KiB direct loads per wave per stage
+    constexpr int CPR = DH / 4;           // 16-byte chunks per row
+    constexpr int HALF = DH / 2;
+    static_assert(DH == 64 || DH == 128, "head dimension 64 or 128");
+    constexpr int FST = fa_stages<DH>();
+    char* const stg[2] = {t0, t1};
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
+
+    const FaItem w = fa_work<DH>(a, item);
+    const int head = w.head, g = w.g, k_lo = w.k_lo, nkb = w.nkb;
 
     const float* __restrict__ Qh = a.q[head];
     const float* __restrict__ Kh = a.k[head];
@@ -208,42 +270,122 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
     }
     wait_vmcnt<0>();  // the trailing zero loads still write LDS
     if (!wave_live) return;
+    fa_store<DH>(a, w, o, m_run, l_run, 1.0f, wave, lane);
+}
 
-    // Row sums: each lane half summed its own 16 keys per block.
-    const float l_tot = l_run + __shfl_xor(l_run, 32);
-    // o[d][4 gg + r] is O[query][32 d + 8 gg + 4 h + r].
-    if (nch == 1) {
-        if (query >= a.seq) return;
-        if (a.lse[head] != nullptr && h == 0) a.lse[head][query] = fa_lse(m_run, l_tot);
-        const float inv = l_tot > 1e-9f ? 1.0f / l_tot : 0.0f;
-        float* orow = a.o[head] + (int64_t)query * DH;
+// The same work item on the bf16 matrix cores (vedic_split.hpp): K and V
+// blocks are split into three bf16 parts as they go from registers to LDS (two
+// buffers, one barrier per 32 keys, the block after next in flight), Q once per
+// item, P in registers.  Per block and wave DH / 16 x 6 MFMAs for S^T and
+// DH / 32 x 2 x 6 for O^T, 32 cycles each, against DH of 64 cycles on
+// v_mfma_f32_32x32x2_f32.  scale log2(e) goes into Q before the split, so the
+// scores come out in base 2; V is scaled by 2^24 (vedic_split.hpp).
+//
+// Returns whether the workgroup's results stand.  They do not if a sum is not
+// finite (an infinity or NaN among the operands, a value of 2^104 or more) or a
+// row's largest score is below -1e28, which the fp32 kernel treats as masked;
+// then nothing has been written and the caller repeats the item with fa_item.
+// (Scores keep the fp32 error for |Q|, |K| < 2^76: values below 2^-126 flush.)
+template <int DH>
+__device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char* b0, char* b1) {
+    constexpr int KB = fs_block_bytes<DH>();
+    constexpr int NT = 256;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const FaItem w = fa_work<DH>(a, item);
+    const float* __restrict__ Kh = a.k[w.head];
+    const float* __restrict__ Vh = a.v[w.head];
+    const int q0 = w.g * kFaQ + 32 * wave;
+    const int query = q0 + l32;
+    const bool wave_live = q0 < a.seq;
+
+    SplitFrag qf[DH / 16];
+    fs_load_rows<DH>(qf, a.q[w.head], query, a.seq, a.scale * 1.4426950408889634f, lane);
+
+    float16_t o[DH / 32];
 #pragma unroll
-        for (int d = 0; d < DH / 32; ++d)
+    for (int d = 0; d < DH / 32; ++d) o[d] = float16_t{};
+    float m_run = kFaMasked, l_run = 0.0f;
+
+    FsAddr<DH> ad(lane);
+    FsStage<DH, NT> sk, sv;
+    auto load = [&](int kb) {  // past the range: zeros, no memory touched
+        const int key0 = w.k_lo + kb * kFaKeys, rows = kb < w.nkb ? a.seq - key0 : 0;
+        sk.load(Kh, key0, rows, tid);
+        sv.load(Vh, key0, rows, tid);
+    };
+    auto commit = [&](char* buf) {
+        sk.commit(buf, 1.0f, tid);
+        sv.commit(buf + KB, kSplitScale, tid);
+    };
+    // Keys key0 .. key0 + 31 in `buf`.
+    auto compute = [&](const char* buf, int key0) {
+        float16_t s = float16_t{};
 #pragma unroll
-            for (int gg = 0; gg < 4; ++gg) {
-                float4_t v;
+        for (int j = 0; j < DH / 16; ++j) s = mfma_split(fs_row<DH>(buf, ad, j), qf[j], s);
+        // s[4 gg + r] is the score of key key0 + 8 gg + 4 h + r for this lane's query.
+        if (a.sparse || key0 + kFaKeys > a.seq || (a.causal && key0 + kFaKeys - 1 > q0)) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = o[d][4 * gg + r] * inv;
-                store16_hold(orow + 32 * d + 8 * gg + 4 * h, v);
-            }
-    } else {
-        // partial slot: [kFaQ][DH] unnormalised O, then the row maxima and sums
-        float* slot = a.part + ((int64_t)head * a.items + asc) * (kFaQ * DH + 2 * kFaQ);
-        float* orow = slot + (int64_t)(32 * wave + l32) * DH;
-#pragma unroll
-        for (int d = 0; d < DH / 32; ++d)
-#pragma unroll
-            for (int gg = 0; gg < 4; ++gg) {
-                float4_t v;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = o[d][4 * gg + r];
-                store16_hold(orow + 32 * d + 8 * gg + 4 * h, v);
-            }
-        if (h == 0) {
-            slot[kFaQ * DH + 32 * wave + l32] = m_run;
-            slot[kFaQ * DH + kFaQ + 32 * wave + l32] = l_tot;
+            for (int i = 0; i < 16; ++i)
+                s[i] = fa_allowed_score(a, s[i], key0 + 8 * (i >> 2) + 4 * h + (i & 3), query);
         }
+        float mx = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        if (__any(mx > m_run)) {  // (a factor of 1 for every row otherwise)
+            const float m_new = fmaxf(m_run, mx);
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int d = 0; d < DH / 32; ++d) o[d] *= alpha;
+        }
+        // (a masked score's exponential is 0, also in a row with no key yet)
+        const float m_ref = m_run == kFaMasked ? 0.0f : m_run;
+        float ls = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = __builtin_amdgcn_exp2f(s[i] - m_ref);
+            ls += s[i];
+        }
+        l_run += ls;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const SplitFrag pf = fs_acc(s, j);
+#pragma unroll
+            for (int d = 0; d < DH / 32; ++d) o[d] = mfma_split(fs_col<DH>(buf + KB, ad, d, j), pf, o[d]);
+        }
+    };
+    // Step kb: block kb is in `cur`, block kb + 1 in registers.
+    auto step = [&](const char* cur, char* nxt, int kb) {
+        const int key0 = w.k_lo + kb * kFaKeys;
+        commit(nxt);
+        load(kb + 2);
+        ad.refresh();
+        // (past the item's keys only for an odd count's last step)
+        if (wave_live && kb < w.nkb && !(a.causal && key0 > q0 + 31) && !(a.sparse && !fa_sparse_any(a, key0, q0)))
+            compute(cur, key0);
+        stage_barrier();
+    };
+
+    load(0);
+    commit(b0);
+    load(1);
+    stage_barrier();
+    for (int kb = 0; kb < w.nkb; kb += 2) {
+        step(b0, b1, kb);
+        step(b1, b0, kb + 1);
     }
+
+    float probe = l_run * 0.0f;
+#pragma unroll
+    for (int d = 0; d < DH / 32; ++d) probe = nonfinite_probe(o[d], probe);
+    const bool bad = probe != 0.0f || (m_run < -1e28f && m_run > kFaMasked);
+    if (__syncthreads_or(bad)) return false;
+    if (wave_live) fa_store<DH>(a, w, o, m_run, l_run, kSplitUnscale, wave, lane);
+    return true;
 }
 
 // One work item per workgroup, or (a.queue set) a grid of resident workgroups
@@ -251,16 +393,27 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
 // so the tail of the key-split one-head case stays balanced.
 // DH 64: registers held to three waves per SIMD, the occupancy its 48 KB of
 // LDS allows (three workgroups per CU); DH 128: two (two 64 KB workgroups).
+template <int DH>
+constexpr bool fa_split() {
+    return DH == 64;
+}
+template <int DH>
+__device__ __forceinline__ void fa_run(const FlashArgs& a, int item, char* b0, char* b1) {
+    if constexpr (fa_split<DH>()) {
+        if (fa_item_split<DH>(a, item, b0, b1)) return;
+    }
+    fa_item<DH>(a, item, b0, b1);
+}
 template <int DH, bool QUEUE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DH == 64 ? 3 : VEDIC_FA_WPE128)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DH == 64 ? VEDIC_FA_WPE64 : VEDIC_FA_WPE128)))
 flash_attn_kernel(FlashArgs a) {
-    constexpr int SB = fa_stage_bytes<DH>();
-    __shared__ __attribute__((aligned(1024))) char t0[SB];
-    __shared__ __attribute__((aligned(1024))) char t1[SB];
-    __shared__ __attribute__((aligned(1024))) char t2[fa_stages<DH>() > 2 ? SB : 16];
+    // two LDS objects: reads of one stage provably do not alias writes of the other
+    constexpr int SB = fa_split<DH>() ? 2 * fs_block_bytes<DH>() : fa_stage_bytes<DH>();
+    __shared__ __attribute__((aligned(1024))) char b0[SB];
+    __shared__ __attribute__((aligned(1024))) char b1[SB];
     __shared__ int next;
     if constexpr (!QUEUE) {
-        fa_item<DH>(a, blockIdx.x, t0, t1, t2);
+        fa_run<DH>(a, blockIdx.x, b0, b1);
         return;
     }
     const int total = a.items * a.nheads;
@@ -270,7 +423,7 @@ flash_attn_kernel(FlashArgs a) {
         const int item = next;
         __syncthreads();  // every wave has its item before `next` is written again
         if (item >= total) break;
-        fa_item<DH>(a, item, t0, t1, t2);
+        fa_run<DH>(a, item, b0, b1);
         __syncthreads();  // every wave is done with the stage buffers
     }
 }

@@ -19,6 +19,15 @@ __device__ __forceinline__ float fa_allowed_score(const Args& a, float s, int ke
     return ok ? s : kFaMasked;
 }
 
+// Whether the sparse mask (a.sparse set) leaves some of keys key0 .. key0 + 31
+// to some of queries q0 .. q0 + 31: a window that reaches them, or a multiple
+// of the stride among them.
+template <class Args>
+__device__ __forceinline__ bool fa_sparse_any(const Args& a, int key0, int q0) {
+    if (key0 + 31 >= q0 - a.window && key0 <= q0 + 31) return true;
+    return (key0 + 31) / a.stride * a.stride >= key0;
+}
+
 // Direct loads of one K block and one V block (keys key0 .. key0 + 31) into
 // stage `dst`: instruction i of this wave fills bytes [1 KiB (wave NLD + i),
 // +1 KiB), lane L its 16-byte chunk L.  Rows at or past `rows` (0 for a

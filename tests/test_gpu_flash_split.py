@@ -1,0 +1,99 @@
+"""Attention on the bf16 matrix cores (three exact bf16 parts per value): what
+the split does not cover is repeated on the fp32 MFMA with the same results as
+binary32 arithmetic -- infinities, NaN, values of 2^104 and more, scores far
+below zero -- and sparse masks whose 32-key blocks have no allowed key."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle import oracle as o  # noqa: E402
+from tests._gpu_helpers import dev, fp32_tol, host, normal  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def vedic():
+    from logos_amd import vedic as v
+
+    return v
+
+
+def _nan_equal(got, want):
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    fin = np.isfinite(want)
+    return fin
+
+
+@pytest.mark.parametrize("seq", [40, 700])
+def test_nonfinite_operands(seq):
+    """One infinite V entry reaches every query that attends to its key (P > 0
+    there), a NaN in Q or K its row or the rows that see it, and the rows
+    before them are the finite call's."""
+    v = vedic()
+    rng = np.random.default_rng(seq)
+    Q, K, V = (normal(rng, (seq, 64)) for _ in range(3))
+    clean = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V)))
+    V2 = V.copy()
+    V2[seq // 2, 5] = np.inf
+    got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V2)))
+    assert np.all(np.isinf(got[seq // 2:, 5]) | np.isnan(got[seq // 2:, 5]))
+    err = np.abs(got[:seq // 2 // 32 * 32] - clean[:seq // 2 // 32 * 32])
+    assert err.size == 0 or err.max() <= fp32_tol(64) * np.abs(clean).max()
+    Q2 = Q.copy()
+    Q2[seq // 3, 7] = np.nan
+    got = host(v.flash_attention_fwd(dev(Q2), dev(K), dev(V)))
+    assert np.all(np.isnan(got[seq // 3]))
+    rest = np.delete(np.arange(seq), seq // 3)
+    assert np.abs(got[rest] - clean[rest]).max() <= fp32_tol(64) * np.abs(clean).max()
+
+
+@pytest.mark.parametrize("heads", [1, 3])
+@pytest.mark.parametrize("scales", [(1.0, 1.0, 2.0 ** 110), (2.0 ** 60, 2.0 ** -60, 2.0 ** -130), (1e-30, 1e-30, 1.0),
+                                    (2.0 ** -126, 2.0 ** 100, 1.0), (3.0, 3.0, 2.0 ** -146)])
+def test_scales(heads, scales):
+    """Q, K and V at extreme scales against float64."""
+    v = vedic()
+    rng = np.random.default_rng(17)
+    seq, dh = 333, 64
+    sq, sk, sv = (np.float32(x) for x in scales)
+    Q, K, V = ([normal(rng, (seq, dh)) * s for _ in range(heads)] for s in (sq, sk, sv))
+    outs = v.flash_attention_fwd_heads([dev(x) for x in Q], [dev(x) for x in K], [dev(x) for x in V])
+    for i in range(heads):
+        want = o.flash_attention_f64(Q[i], K[i], V[i], 0.125, 1, 0, 0, 1)
+        # subnormal results: the partial of each of at most three key chunks and the
+        # merged row are rounded to half of 2^-149
+        assert np.abs(host(outs[i]) - want).max() <= fp32_tol(dh) * np.abs(want).max() + 4 * 2.0 ** -150
+
+
+def test_scores_far_below_zero():
+    """Rows whose every score is about -2^101: below -1e29 the reference counts
+    a score as masked."""
+    v = vedic()
+    rng = np.random.default_rng(19)
+    seq, dh = 70, 64
+    Q, K, V = np.abs(normal(rng, (seq, dh))), -np.abs(normal(rng, (seq, dh))), normal(rng, (seq, dh))
+    Q[10:20] *= np.float32(2.0 ** 101)
+    got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V)))
+    want = o.flash_attention(Q, K, V, 0.125, 1, 0, 0, 1)
+    assert np.all(got[10:20] == 0) and np.all(want[10:20] == 0)
+    rest = np.r_[0:10, 20:seq]
+    assert np.abs(got[rest] - want[rest]).max() <= 2 * fp32_tol(dh) * np.abs(want[rest]).max()
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("window,stride", [(0, 1000), (31, 33), (32, 64), (100, 129), (5, 32)])
+def test_sparse_blocks(causal, window, stride):
+    """Windows and strides around the 32-key block: whole blocks with no
+    allowed key for a wave's 32 queries, and blocks with one."""
+    v = vedic()
+    rng = np.random.default_rng(window * 1000 + stride)
+    seq, dh = 419, 64
+    Q, K, V = (normal(rng, (seq, dh)) for _ in range(3))
+    lse = torch.empty(seq, device="cuda")
+    kw = dict(causal=bool(causal), shunyam=True, window=window, stride=stride)
+    got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V), lse=lse, **kw))
+    want = o.flash_attention_f64(Q, K, V, 0.125, causal, 1, window, stride)
+    assert o.inf_rel_err(got, want) <= fp32_tol(dh)
