@@ -1,4 +1,5 @@
-// vedic_flash_attn.hip -- fused attention forward for gfx950, fp32 throughout.
+// vedic_flash_attn.hip -- fused attention forward for gfx950, fp32 in and out
+// (DH 64 on the bf16 matrix cores by exact splits, fa_item_split).
 //
 //   out = softmax(scale * Q . K^T + mask) . V          per head, Q/K/V/out [seq x DH]
 //
@@ -278,7 +279,9 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
 // buffers, one barrier per 32 keys, the block after next in flight), Q once per
 // item, P in registers.  Per block and wave DH / 16 x 6 MFMAs for S^T and
 // DH / 32 x 2 x 6 for O^T, 32 cycles each, against DH of 64 cycles on
-// v_mfma_f32_32x32x2_f32.  scale log2(e) goes into Q before the split, so the
+// v_mfma_f32_32x32x2_f32: 16 heads x seq 8192 causal 1213 -> 688-726 us, the
+// matrix pipe 62 % busy at 1.72 GHz, 6 VALU instructions (split, softmax) per
+// MFMA beside it.  scale log2(e) goes into Q before the split, so the
 // scores come out in base 2; V is scaled by 2^24 (vedic_split.hpp).
 //
 // Returns whether the workgroup's results stand.  They do not if a sum is not

@@ -1,4 +1,5 @@
-// vedic_flash_attn_bwd.hip -- fused attention backward for gfx950, fp32.
+// vedic_flash_attn_bwd.hip -- fused attention backward for gfx950, fp32 in and
+// out (DH 64 on the bf16 matrix cores by exact splits, see the end).
 //
 // Given Q, K, V, the forward output O, its gradient dO and the forward's
 // per-row log-sum-exp lse (vedic_flash_attention_fwd_lse), computes
@@ -34,6 +35,7 @@
 #include <hip/hip_runtime.h>
 
 #include "vedic_flash_device.hpp"
+#include "vedic_flash_split.hpp"
 
 namespace vedic {
 
@@ -92,35 +94,22 @@ __device__ __forceinline__ bool fb_masked(const A& a, int key, int query) {
 
 // ------------------------------------------------------------------ dQ pass
 
-// DH 128: two stages instead of three.  The passes stay at one wave per SIMD
-// (370-453 registers), but the small spills of the dQ pass and the dK launch
-// go away: 8 heads x seq 8192 5636 -> 5459 us.  (Two waves per SIMD would cap
-// them at 256 registers: 280-650 bytes of scratch per lane.)
-#ifndef VEDIC_FB_ST128
-#define VEDIC_FB_ST128 2
-#endif
+// (At DH 128 the passes run at one wave per SIMD, 370-453 registers; two waves
+// per SIMD would cap them at 256: 280-650 bytes of scratch per lane.)
 #ifndef VEDIC_FB_WPE128
 #define VEDIC_FB_WPE128 1
 #endif
-// LDS stages in flight of the backward passes
-template <int DH>
-constexpr int fb_stages() {
-    return DH == 128 ? VEDIC_FB_ST128 : kFaStages;
-}
+constexpr int kFbStages = 2;  // LDS stages in flight of the fp32 passes
 
 template <int DH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DH == 64 ? 2 : VEDIC_FB_WPE128)))
-flash_bwd_dq_kernel(FlashBwdArgs a) {
+__device__ __forceinline__ void fb_dq_item(const FlashBwdArgs& a, int item, char* t0, char* t1) {
     constexpr int KB = 32 * DH * 4, SB = 2 * KB, NLD = SB / 1024 / 4, HALF = DH / 2;
-    constexpr int FST = fb_stages<DH>();
-    __shared__ __attribute__((aligned(1024))) char t0[SB];
-    __shared__ __attribute__((aligned(1024))) char t1[SB];
-    __shared__ __attribute__((aligned(1024))) char t2[FST > 2 ? SB : 16];
-    char* const stg[3] = {t0, t1, t2};
+    constexpr int FST = kFbStages;
+    char* const stg[2] = {t0, t1};
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
-    const int head = blockIdx.x % a.nheads;
-    const int g = a.nqg - 1 - (int)(blockIdx.x / a.nheads);  // largest key ranges first
+    const int head = item % a.nheads;
+    const int g = a.nqg - 1 - item / a.nheads;  // largest key ranges first
     const int q0 = g * kFaQ + 32 * wave, query = q0 + l32;
     const int kend = a.causal ? min(a.seq, kFaQ * (g + 1)) : a.seq;
     const int nkb = (kend + 31) / 32;
@@ -235,25 +224,20 @@ flash_bwd_dq_kernel(FlashBwdArgs a) {
 
 // --------------------------------------------------------------- dK/dV pass
 
-// PART 0: dK and dV together.  At DH 128 the two do not fit one wave's
-// registers beside K and V (168 registers spilled), so they run as two
-// launches: PART 1 dV only (no V, no dP), PART 2 dK only; the second
-// recomputes S (five products per block instead of four) but nothing spills.
-template <int DH, int PART = 0>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DH == 64 ? 1 : VEDIC_FB_WPE128)))
-flash_bwd_dkdv_kernel(FlashBwdArgs a) {
+// PART 1: dV only (no V, no dP); PART 2: dK only.  Together they do not fit
+// one wave's registers beside K and V at DH 128; the second recomputes S (five
+// products per block instead of four) but nothing spills.
+template <int DH, int PART>
+__device__ __forceinline__ void fb_dkdv_item(const FlashBwdArgs& a, int item, char* t0, char* t1) {
     constexpr int KB = 32 * DH * 4, NLD = 2 * KB / 1024 / 4, HALF = DH / 2;
     constexpr bool DO_DV = PART != 2, DO_DK = PART != 1;
-    constexpr int SB = 2 * KB + 1024;  // Q block, dO block, then (lse2, D) of the 32 queries
-    constexpr int FST = fb_stages<DH>();
-    __shared__ __attribute__((aligned(1024))) char t0[SB];
-    __shared__ __attribute__((aligned(1024))) char t1[SB];
-    __shared__ __attribute__((aligned(1024))) char t2[FST > 2 ? SB : 16];
-    char* const stg[3] = {t0, t1, t2};
+    // a stage: Q block, dO block, then (lse2, D) of the 32 queries
+    constexpr int FST = kFbStages;
+    char* const stg[2] = {t0, t1};
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
-    const int head = blockIdx.x % a.nheads;
-    const int g = (int)(blockIdx.x / a.nheads);  // causal: the first key groups see the most queries
+    const int head = item % a.nheads;
+    const int g = item / a.nheads;  // causal: the first key groups see the most queries
     const int k0 = g * kFaQ + 32 * wave, key = k0 + l32;
     const int qstart = a.causal ? (g * kFaQ) / 32 : 0;
     const int nqb = (a.seq + 31) / 32 - qstart;
@@ -390,11 +374,317 @@ flash_bwd_dkdv_kernel(FlashBwdArgs a) {
         }
 }
 
+// ----------------------------------------------- on the bf16 matrix cores
+
+// Both passes at DH 64 with every operand split exactly into three bf16 parts
+// (vedic_split.hpp): the streamed blocks once per workgroup on their way into
+// LDS (two buffers, one barrier per 32 rows), the resident rows once per item,
+// P and dS in registers.  K, V and dO carry the factor 2^24 of the split, Q
+// (dK/dV pass) too; scale log2(e) 2^-24 goes into the other side of the score
+// product, so scores come out in base 2; dP, D and dS carry 2^48 and the
+// accumulators 2^72 (dV: P is not scaled, 2^24).
+//
+// Bound: the matrix cores, 72 and 96 MFMAs of 32 cycles per 32 x 32 block
+// (fp32: 96 and 128 of 64).  16 heads x seq 8192 causal 4253 -> 2303 us per
+// backward (error against float64 2.2e-6 -> 1.6e-6): 61 and 60 % of the matrix
+// pipe busy at two waves per SIMD (231 and 254 registers), at the 1.83 GHz the
+// chip holds under this load.
+//
+// As in the forward, an item whose sums are not finite is repeated on the
+// fp32 MFMA (with nothing written before but the same lse2 and D).  Scores
+// keep the fp32 error for |Q|, |K| < 2^76.
+constexpr float kFbScale2 = kSplitScale * kSplitScale;  // 2^48
+constexpr float kFbUnscale3 = kSplitUnscale2 * kSplitUnscale;  // 2^-72
+
+template <int DH>
+__device__ __forceinline__ bool fb_dq_split(const FlashBwdArgs& a, int item, char* b0, char* b1) {
+    constexpr int KB = fs_block_bytes<DH>(), NT = 256;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int head = item % a.nheads;
+    const int g = a.nqg - 1 - item / a.nheads;  // largest key ranges first
+    const int q0 = g * kFaQ + 32 * wave, query = q0 + l32;
+    const int kend = a.causal ? min(a.seq, kFaQ * (g + 1)) : a.seq;
+    const int nkb = (kend + 31) / 32;
+    const bool live = q0 < a.seq;
+
+    SplitFrag qf[DH / 16], df[DH / 16];
+    fs_load_rows<DH>(qf, a.q[head], query, a.seq, a.scale * (1.4426950408889634f * kSplitUnscale), lane);
+    float dsum = 0.0f;
+    {
+        const __amdgpu_buffer_rsrc_t rd = buffer_rsrc(a.dout[head]), ro = buffer_rsrc(a.o[head]);
+        const uint32_t off = query < a.seq ? (uint32_t)(query * DH * 4 + h * 32) : kOob;
+#pragma unroll
+        for (int j = 0; j < DH / 16; ++j) {
+            float w[8];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int o = (int)(off == kOob ? kOob : off + 64 * j + 16 * q);
+                const float4_t vd = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rd, o, 0, 0));
+                const float4_t vo = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(ro, o, 0, 0));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    w[4 * q + e] = vd[e] * kSplitScale;
+                    dsum = __builtin_fmaf(vd[e], vo[e], dsum);
+                }
+            }
+            df[j] = split8(w);
+        }
+    }
+    const float D = dsum + __shfl_xor(dsum, 32);
+    const float lse2 = ld_f32(buffer_rsrc(a.lse[head]), query < a.seq ? (uint32_t)query * 4 : kOob, 0) *
+                       1.4426950408889634f;
+    if (live && query < a.seq && h == 0) {
+        float* st = a.delta + ((int64_t)head * a.seq + query) * 2;
+        st[0] = lse2;
+        st[1] = D;
+    }
+    const float D2 = D * kFbScale2;
+
+    float16_t dq[DH / 32];
+#pragma unroll
+    for (int d = 0; d < DH / 32; ++d) dq[d] = float16_t{};
+    FsAddr<DH> ad(lane);
+    FsStage<DH, NT> sk, sv;
+    auto load = [&](int kb) {  // past the range: zeros, no memory touched
+        const int rows = kb < nkb ? a.seq - kb * 32 : 0;
+        sk.load(a.k[head], kb * 32, rows, tid);
+        sv.load(a.v[head], kb * 32, rows, tid);
+    };
+    auto commit = [&](char* buf) {
+        sk.commit(buf, kSplitScale, tid);
+        sv.commit(buf + KB, kSplitScale, tid);
+    };
+    auto compute = [&](const char* buf, int key0) {
+        float16_t s = float16_t{}, dp = float16_t{};
+#pragma unroll
+        for (int j = 0; j < DH / 16; ++j) s = mfma_split(fs_row<DH>(buf, ad, j), qf[j], s);
+#pragma unroll
+        for (int j = 0; j < DH / 16; ++j) dp = mfma_split(fs_row<DH>(buf + KB, ad, j), df[j], dp);
+        // s[4 gg + r]: key key0 + 8 gg + 4 h + r of this lane's query
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(s[i] - lse2);
+        if (a.sparse || key0 + 32 > a.seq || (a.causal && key0 + 31 > q0)) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                s[i] = fa_allowed_score(a, s[i], key0 + 8 * (i >> 2) + 4 * h + (i & 3), query) == kFaMasked ? 0.0f : s[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] *= dp[i] - D2;  // dS^T
+        // dQ^T[d][q] += sum over keys K[key][d] dS^T[key][q]
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const SplitFrag sf = fs_acc(s, j);
+#pragma unroll
+            for (int d = 0; d < DH / 32; ++d) dq[d] = mfma_split(fs_col<DH>(buf, ad, d, j), sf, dq[d]);
+        }
+    };
+    auto step = [&](const char* cur, char* nxt, int kb) {
+        const int key0 = kb * 32;
+        commit(nxt);
+        load(kb + 2);
+        ad.refresh();
+        if (live && kb < nkb && !(a.causal && key0 > q0 + 31) && !(a.sparse && !fa_sparse_any(a, key0, q0)))
+            compute(cur, key0);
+        stage_barrier();
+    };
+    load(0);
+    commit(b0);
+    load(1);
+    stage_barrier();
+    for (int kb = 0; kb < nkb; kb += 2) {
+        step(b0, b1, kb);
+        step(b1, b0, kb + 1);
+    }
+
+    float probe = 0.0f;
+#pragma unroll
+    for (int d = 0; d < DH / 32; ++d) probe = nonfinite_probe(dq[d], probe);
+    if (__syncthreads_or(probe != 0.0f)) return false;
+    if (!live || query >= a.seq) return true;
+    const float f = a.scale * kFbUnscale3;
+    float* row = a.dq[head] + (int64_t)query * DH;
+#pragma unroll
+    for (int d = 0; d < DH / 32; ++d)
+#pragma unroll
+        for (int gg = 0; gg < 4; ++gg) {
+            float4_t v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = dq[d][4 * gg + r] * f;
+            store16_hold(row + 32 * d + 8 * gg + 4 * h, v);
+        }
+    return true;
+}
+
+// A stage of the dK/dV pass: the Q block, the dO block, then lse2[32] and
+// D[32] of the queries (+inf and 0 past seq: P and dS are 0 there).
+template <int DH>
+constexpr int fb_split_stage_bytes() {
+    return 2 * fs_block_bytes<DH>() + 256;
+}
+
+template <int DH>
+__device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, char* b0, char* b1) {
+    constexpr int KB = fs_block_bytes<DH>(), NT = 256;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int head = item % a.nheads;
+    const int g = item / a.nheads;  // causal: the first key groups see the most queries
+    const int k0 = g * kFaQ + 32 * wave, key = k0 + l32;
+    const int qstart = a.causal ? (g * kFaQ) / 32 : 0;
+    const int nqb = (a.seq + 31) / 32 - qstart;
+    const bool live = k0 < a.seq;
+
+    SplitFrag kf[DH / 16], vf[DH / 16];
+    fs_load_rows<DH>(kf, a.k[head], key, a.seq, a.scale * (1.4426950408889634f * kSplitUnscale), lane);
+    fs_load_rows<DH>(vf, a.v[head], key, a.seq, kSplitScale, lane);
+    const float* stats = a.delta + (int64_t)head * a.seq * 2;
+
+    float16_t dv[DH / 32], dk[DH / 32];
+#pragma unroll
+    for (int d = 0; d < DH / 32; ++d) {
+        dv[d] = float16_t{};
+        dk[d] = float16_t{};
+    }
+    FsAddr<DH> ad(lane);
+    FsStage<DH, NT> sq, sd;
+    float st = 0.0f;  // threads 0 .. 63: the block's lse2 and D, interleaved
+    auto load = [&](int qb) {
+        const int q0 = (qstart + qb) * 32, rows = qb < nqb ? a.seq - q0 : 0;
+        sq.load(a.q[head], q0, rows, tid);
+        sd.load(a.dout[head], q0, rows, tid);
+        const bool in = tid < 64 && (tid >> 1) < rows;
+        st = ld_f32(buffer_rsrc(stats + (rows > 0 ? (int64_t)q0 * 2 : 0)), in ? (uint32_t)tid * 4 : kOob, 0);
+        st = in ? (tid & 1 ? st * kFbScale2 : st) : tid & 1 ? 0.0f : __builtin_inff();
+    };
+    auto commit = [&](char* buf) {
+        sq.commit(buf, kSplitScale, tid);
+        sd.commit(buf + KB, kSplitScale, tid);
+        if (tid < 64) *reinterpret_cast<float*>(buf + 2 * KB + (tid & 1) * 128 + (tid >> 1) * 4) = st;
+    };
+    auto compute = [&](const char* buf, int qb0) {
+        const char* sl = buf + 2 * KB + 16 * h;
+        float16_t s = float16_t{};
+#pragma unroll
+        for (int j = 0; j < DH / 16; ++j) s = mfma_split(fs_row<DH>(buf, ad, j), kf[j], s);
+        // s[4 gg + r]: query qb0 + 8 gg + 4 h + r against this lane's key
+#pragma unroll
+        for (int gg = 0; gg < 4; ++gg) {
+            const float4_t lse2 = *reinterpret_cast<const float4_t*>(sl + 32 * gg);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[4 * gg + r] = __builtin_amdgcn_exp2f(s[4 * gg + r] - lse2[r]);
+        }
+        if (a.sparse || (a.causal && qb0 < k0 + 31)) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                s[i] = fa_allowed_score(a, s[i], key, qb0 + 8 * (i >> 2) + 4 * h + (i & 3)) == kFaMasked ? 0.0f : s[i];
+        }
+        // dV^T[d][key] += sum over queries dO[q][d] P[q][key]
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const SplitFrag pf = fs_acc(s, j);
+#pragma unroll
+            for (int d = 0; d < DH / 32; ++d) dv[d] = mfma_split(fs_col<DH>(buf + KB, ad, d, j), pf, dv[d]);
+        }
+        float16_t dp = float16_t{};
+#pragma unroll
+        for (int j = 0; j < DH / 16; ++j) dp = mfma_split(fs_row<DH>(buf + KB, ad, j), vf[j], dp);
+#pragma unroll
+        for (int gg = 0; gg < 4; ++gg) {
+            const float4_t D2 = *reinterpret_cast<const float4_t*>(sl + 128 + 32 * gg);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[4 * gg + r] *= dp[4 * gg + r] - D2[r];  // dS
+        }
+        // dK^T[d][key] += sum over queries Q[q][d] dS[q][key]
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const SplitFrag sf = fs_acc(s, j);
+#pragma unroll
+            for (int d = 0; d < DH / 32; ++d) dk[d] = mfma_split(fs_col<DH>(buf, ad, d, j), sf, dk[d]);
+        }
+    };
+    auto step = [&](const char* cur, char* nxt, int qb) {
+        const int qb0 = (qstart + qb) * 32;
+        commit(nxt);
+        load(qb + 2);
+        ad.refresh();
+        if (live && qb < nqb && !(a.causal && qb0 + 31 < k0) && !(a.sparse && !fa_sparse_any(a, k0, qb0))) compute(cur, qb0);
+        stage_barrier();
+    };
+    load(0);
+    commit(b0);
+    load(1);
+    stage_barrier();
+    for (int qb = 0; qb < nqb; qb += 2) {
+        step(b0, b1, qb);
+        step(b1, b0, qb + 1);
+    }
+
+    float probe = 0.0f;
+#pragma unroll
+    for (int d = 0; d < DH / 32; ++d) probe = nonfinite_probe(dk[d], nonfinite_probe(dv[d], probe));
+    // (keys past seq are not stored: their sums may be anything)
+    if (__syncthreads_or(key < a.seq && probe != 0.0f)) return false;
+    if (!live || key >= a.seq) return true;
+    const float f = a.scale * kFbUnscale3;
+    float* vrow = a.dv[head] + (int64_t)key * DH;
+    float* krow = a.dk[head] + (int64_t)key * DH;
+#pragma unroll
+    for (int d = 0; d < DH / 32; ++d)
+#pragma unroll
+        for (int gg = 0; gg < 4; ++gg) {
+            float4_t v, w;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v[r] = dv[d][4 * gg + r] * kSplitUnscale;
+                w[r] = dk[d][4 * gg + r] * f;
+            }
+            store16_hold(vrow + 32 * d + 8 * gg + 4 * h, v);
+            store16_hold(krow + 32 * d + 8 * gg + 4 * h, w);
+        }
+    return true;
+}
+
+#ifndef VEDIC_FB_DQ_WPE
+#define VEDIC_FB_DQ_WPE 2
+#endif
+template <int DH>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(DH == 64 ? VEDIC_FB_DQ_WPE : VEDIC_FB_WPE128))) flash_bwd_dq_kernel(FlashBwdArgs a) {
+    constexpr int SB = DH == 64 ? 2 * fs_block_bytes<DH>() : 2 * 32 * DH * 4;
+    __shared__ __attribute__((aligned(1024))) char t0[SB];
+    __shared__ __attribute__((aligned(1024))) char t1[SB];
+    if constexpr (DH == 64) {
+        if (fb_dq_split<DH>(a, blockIdx.x, t0, t1)) return;
+    }
+    fb_dq_item<DH>(a, blockIdx.x, t0, t1);
+}
+
+// PART 0 (DH 64): dK and dV together on the split, each on its own in the
+// repeat; PART 1 and 2 (DH 128): dV and dK.
+template <int DH, int PART>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DH == 64 ? 2 : VEDIC_FB_WPE128)))
+flash_bwd_dkdv_kernel(FlashBwdArgs a) {
+    constexpr int SB = DH == 64 ? fb_split_stage_bytes<DH>() : 2 * 32 * DH * 4 + 1024;
+    __shared__ __attribute__((aligned(1024))) char t0[SB];
+    __shared__ __attribute__((aligned(1024))) char t1[SB];
+    if constexpr (PART == 0) {
+        if (fb_dkdv_split<DH>(a, blockIdx.x, t0, t1)) return;
+        fb_dkdv_item<DH, 1>(a, blockIdx.x, t0, t1);
+        __syncthreads();  // every wave is done with the stage buffers
+        fb_dkdv_item<DH, 2>(a, blockIdx.x, t0, t1);
+    } else {
+        fb_dkdv_item<DH, PART>(a, blockIdx.x, t0, t1);
+    }
+}
+
 hipError_t launch_flash_attn_bwd(const FlashBwdArgs& a, int dh, hipStream_t s) {
     const dim3 grid((unsigned)(a.nqg * a.nheads));
     if (dh == 64) {
         hipLaunchKernelGGL(flash_bwd_dq_kernel<64>, grid, dim3(256), 0, s, a);
-        hipLaunchKernelGGL(flash_bwd_dkdv_kernel<64>, grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((flash_bwd_dkdv_kernel<64, 0>), grid, dim3(256), 0, s, a);
     } else {
         hipLaunchKernelGGL(flash_bwd_dq_kernel<128>, grid, dim3(256), 0, s, a);
         hipLaunchKernelGGL((flash_bwd_dkdv_kernel<128, 1>), grid, dim3(256), 0, s, a);

@@ -97,3 +97,55 @@ def test_sparse_blocks(causal, window, stride):
     got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V), lse=lse, **kw))
     want = o.flash_attention_f64(Q, K, V, 0.125, causal, 1, window, stride)
     assert o.inf_rel_err(got, want) <= fp32_tol(dh)
+
+
+def _backward(v, Q, K, V, dO, **kw):
+    tQ, tK, tV = dev(Q), dev(K), dev(V)
+    lse = torch.empty(Q.shape[0], device="cuda")
+    out = v.flash_attention_fwd(tQ, tK, tV, lse=lse, **kw)
+    return tuple(host(t) for t in v.flash_attention_bwd(tQ, tK, tV, out, dev(dO), lse, **kw))
+
+
+@pytest.mark.parametrize("scales", [(1.0, 1.0, 1.0, 2.0 ** -60), (1.0, 1.0, 2.0 ** 50, 2.0 ** 40), (1e-20, 1e-20, 1.0, 1.0),
+                                    (2.0 ** 30, 2.0 ** -30, 1.0, 1.0), (1.0, 1.0, 2.0 ** -70, 2.0 ** 20)])
+def test_backward_scales(scales):
+    """Operands and gradients at extreme scales: within the split's range, past
+    its scaled sums (repeated on the fp32 MFMA) and below bf16's normal range."""
+    v = vedic()
+    rng = np.random.default_rng(23)
+    seq, dh = 205, 64
+    Q, K, V, dO = (normal(rng, (seq, dh)) * np.float32(s) for s in scales)
+    got = _backward(v, Q, K, V, dO)
+    want = o.flash_attention_bwd_f64(Q, K, V, dO, 0.125)
+    for g, w, name in zip(got, want, ("dQ", "dK", "dV")):
+        assert np.abs(g - w).max() <= fp32_tol(seq) * np.abs(w).max(), name
+
+
+def test_backward_nonfinite():
+    """A NaN in one dO row reaches every dK, dV row it attends to and its own
+    dQ row; the other queries keep their finite dQ and the keys past its
+    32-key block (whose masked weights of 0 meet the NaN) their dV."""
+    v = vedic()
+    rng = np.random.default_rng(29)
+    seq, dh = 300, 64
+    Q, K, V, dO = (normal(rng, (seq, dh)) for _ in range(4))
+    clean = _backward(v, Q, K, V, dO)
+    dO2 = dO.copy()
+    dO2[200, 3] = np.nan
+    dQ, dK, dV = _backward(v, Q, K, V, dO2)
+    assert np.all(np.isnan(dQ[200])) and np.all(np.isnan(dV[:201, 3])) and np.all(np.isnan(dK[:201]))
+    rest = np.delete(np.arange(seq), 200)
+    assert np.abs(dQ[rest] - clean[0][rest]).max() <= fp32_tol(seq) * np.abs(clean[0]).max()
+    assert np.abs(dV[224:] - clean[2][224:]).max() <= fp32_tol(seq) * np.abs(clean[2]).max()
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("window,stride", [(0, 1000), (31, 33), (100, 129)])
+def test_backward_sparse_blocks(causal, window, stride):
+    v = vedic()
+    rng = np.random.default_rng(window * 1000 + stride + 1)
+    seq, dh = 419, 64
+    Q, K, V, dO = (normal(rng, (seq, dh)) for _ in range(4))
+    got = _backward(v, Q, K, V, dO, causal=bool(causal), shunyam=True, window=window, stride=stride)
+    want = o.flash_attention_bwd_f64(Q, K, V, dO, 0.125, causal, 1, window, stride)
+    assert o.grad_rel_err(got, want) <= fp32_tol(seq)
