@@ -212,12 +212,13 @@ int vedic_gemm_bias_gelu_f32(const float* X, const float* W, const float* bias, 
  * casts the activation on every call, cuda/ModelGPU.cu:825-827); fp32
  * accumulation and output.  When W16 is NULL the call is the fp32 product
  * with W32, as the reference falls back to cuda_vedic_gemm(_bias) for a
- * parameter without a shadow.  A and C contiguous.  For N > 1024, or an A
- * whose base is not 16-byte aligned or whose K is not a multiple of 8, the
- * call casts A into an M x K binary16 workspace (the stream's workspace
- * block) and runs the fp16 GEMM on it: each output tile converts its
- * own rows of A, ceil(N / 128) conversions per element, which loses to one
- * cast pass for wide products.  Results are the same bits either way. */
+ * parameter without a shadow.  A and C contiguous.  For N > 1024, for
+ * N > 512 with K >= 2048 and M > 32, or an A whose base is not 16-byte aligned
+ * or whose K is not a multiple of 8, the call casts A into an M x K binary16
+ * workspace (the stream's workspace block) and runs the fp16 GEMM on it: each
+ * output tile reads and converts its own rows of the fp32 A, ceil(N / 128)
+ * times per element, which loses to one cast pass for wide products.  Results
+ * are the same bits either way. */
 int vedic_amp_gemm(const float* A, int M, int K, const void* W16, const float* W32, int N, float* C,
                    void* stream);
 int vedic_amp_gemm_bias(const float* A, int M, int K, const void* W16, const float* W32, int N,

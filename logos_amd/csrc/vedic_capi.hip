@@ -67,8 +67,6 @@ static int hip_status(hipError_t e) {
 
 static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
-// Largest leading dimension (elements) the kernels' 32-bit tile offsets allow.
-
 // Temporary device memory of library calls (split-K partial slabs, column
 // partials, the AMP cast buffer, attention partials and padded copies) comes
 // from an arena per (device, stream): grown on demand and kept for the next
@@ -192,7 +190,12 @@ struct Workspace {
             a->mu.lock();
             arena = a;
             mark = a->used;
-            if (a->used == 0 && a->want > a->cap) {
+            // (not inside a stream capture: the block would belong to the graph;
+            // its pieces come from the pool, as nodes of the graph)
+            hipStreamCaptureStatus cap_status = hipStreamCaptureStatusNone;
+            if (a->used == 0 && a->want > a->cap &&
+                (s == nullptr || hipStreamIsCapturing(s, &cap_status) != hipSuccess ||
+                 cap_status == hipStreamCaptureStatusNone)) {
                 // grow (the old block is freed after the work queued on it)
                 if (a->base) (void)hipFreeAsync(a->base, s);
                 a->base = nullptr;
@@ -503,6 +506,16 @@ constexpr int kOpAmp = 3;
 #define VEDIC_AMP_IN_KERNEL_MAX_N 1024
 #endif
 constexpr int kAmpInKernelMaxN = VEDIC_AMP_IN_KERNEL_MAX_N;
+// Long contractions of more than 512 columns take the cast too: every tile
+// column reads the fp32 A again, and its 4 bytes per value bound the stages
+// (1531 x 1024 x 4096 41.3 us in the kernel, 6.7 + 25.5 cast + binary16 GEMM;
+// 8192 x 1024 x 4096 98.8, 27.8 + 67.6; but 512 x 1024 x 1024 17.9, 6.6 + 11.8,
+// and 4096 x 512 x 2048 27.5, 8.3 + 21.2).
+// (M <= 32 after the cast would run on the decode kernel, whose sums have
+// another order than the in-kernel conversion's.)
+static bool amp_cast_first(int M, int N, int K) {
+    return N > kAmpInKernelMaxN || (M > 32 && N > 512 && K >= 2048);
+}
 
 static hipError_t launch_f16_direct(int op, const GemmArgs& a, hipStream_t s) {
     return op == VEDIC_OP_NN   ? launch_gemm_f16_direct_nn(a, s)
@@ -691,7 +704,10 @@ static int gemm_impl(const vedic_gemm_desc_t* d, float* const* heads, int nheads
     const bool f16 = d->in_dtype != VEDIC_DT_F32;
     // (an fp32 A's tile rows are twice as long in bytes)
     const bool direct = vec && d->lda < (amp ? kMaxLd / 2 : kMaxLd) && d->ldb < kMaxLd;
-    if (amp && (!direct || d->N > kAmpInKernelMaxN)) return amp_via_cast(d, heads, nheads, head_cols, handoff, wsp);
+    // (a caller's fixed scratch region is asked for a copy of A only where it
+    // must: the bits are the same)
+    if (amp && (!direct || (wsp ? d->N > kAmpInKernelMaxN : amp_cast_first(d->M, d->N, d->K))))
+        return amp_via_cast(d, heads, nheads, head_cols, handoff, wsp);
     // scattered C needs the kernels with a plain or bias epilogue kind
     if (scatter && !direct) return VEDIC_STATUS_BAD_LD;
     const bool skinny = direct && !amp && d->op == VEDIC_OP_NN && d->M <= 32;

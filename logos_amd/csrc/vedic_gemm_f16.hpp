@@ -146,7 +146,31 @@ struct Side {
     }
 };
 
-// An fp32 A operand stored [M x K] (k contiguous) for the AMP path: each
+// Eight values as binary16: rounded to nearest even first (packed, two values
+// per instruction), then the pairs clamped to +-65504 (packed min/max, IEEE
+// minNum / maxNum): the same bits as clamping in fp32 first.  Finite values at
+// or above 65520 round to infinity and clamp back to 65504; values below it
+// round to at most 65504; infinities clamp; a NaN converts to a NaN, which
+// minNum replaces by 65504, as fminf does in the fp32 clamp.
+__device__ __forceinline__ half8_t half8_clamped(const float4_t& a, const float4_t& b) {
+    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    const half2_t hi = {(_Float16)65504.0f, (_Float16)65504.0f};
+    const half2_t lo = {(_Float16)-65504.0f, (_Float16)-65504.0f};
+    half8_t hv;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const f32x2_t f = e < 4 ? f32x2_t{a[e & 3], a[(e & 3) + 1]} : f32x2_t{b[e & 3], b[(e & 3) + 1]};
+        half2_t h = __builtin_convertvector(f, half2_t);
+        h = __builtin_elementwise_max(__builtin_elementwise_min(h, hi), lo);
+        hv[e] = h[0];
+        hv[e + 1] = h[1];
+    }
+    return hv;
+}
+
+// An fp32 A operand stored [M x K] (k contiguous) for the AMP path on the
+// 256 x 128 and the narrow tiles (SideA32D serves the 128 x 128 ones): each
 // 16-byte binary16 chunk of the KC layout is loaded as its eight fp32 values
 // (two 16-byte register loads), clamped and rounded to binary16
 // (to_half_clamped, the cast kernel's conversion) and written to its swizzled
@@ -191,32 +215,52 @@ struct SideA32 {
                                                            rs, (int)(o == kOob ? kOob : o + 16 * h), 0, 0));
         }
     }
-    // Round to nearest even first (packed, two values per instruction), then
-    // clamp the binary16 pair to +-65504 (packed min/max, IEEE minNum /
-    // maxNum): the same bits as clamping in fp32 first.  Finite values at or
-    // above 65520 round to infinity and clamp back to 65504; values below it
-    // round to at most 65504; infinities clamp; a NaN converts to a NaN, which
-    // minNum replaces by 65504, as fminf does in the fp32 clamp.
     __device__ __forceinline__ void commit(char* lds, int wave, int lane) const {
-        typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-        typedef float float2_t __attribute__((ext_vector_type(2)));
-        const half2_t hi = {(_Float16)65504.0f, (_Float16)65504.0f};
-        const half2_t lo = {(_Float16)-65504.0f, (_Float16)-65504.0f};
 #pragma unroll
         for (int i = 0; i < NCH; ++i) {
             int row, p;
             geom(wave, lane, i, row, p);
-            half8_t hv;
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const float2_t f = {v[i][e >> 2][e & 3], v[i][e >> 2][(e & 3) + 1]};
-                half2_t h = __builtin_convertvector(f, half2_t);
-                h = __builtin_elementwise_max(__builtin_elementwise_min(h, hi), lo);
-                hv[e] = h[0];
-                hv[e + 1] = h[1];
-            }
-            *reinterpret_cast<half8_t*>(lds + row * (CPR * 16) + ((p ^ swz_kc<CPR>(row)) << 4)) = hv;
+            *reinterpret_cast<half8_t*>(lds + row * (CPR * 16) + ((p ^ swz_kc<CPR>(row)) << 4)) =
+                half8_clamped(v[i][0], v[i][1]);
         }
+    }
+};
+
+// An fp32 A operand stored [M x K] on its way through LDS as fp32, converted as
+// fragments are read (read_frag_a32): the loads are direct ones like the
+// binary16 operands', so whole stages are in flight.  (SideA32's register loads
+// have one stage's MFMAs to arrive in.)  For 128 x 128 tiles, whose three
+// 48 KiB stages fit LDS: 2000 x 1024 x 1024 20.2 -> 18.4 us, 4096 x 512 x 2048
+// 28.8 -> 27.5, gathered 2000 x 1024 x 1024 25.5 -> 24.1; what bounds it then
+// is the 48 KiB of operands per stage, at the rate the L2 gives each CU (a
+// binary16 A, 32 KiB: 12.1 us).  256 x 128 tiles take 80 KiB per stage; with
+// 32-deep stages they lost (gathered 8192 x 1024 x 1024 35.2 -> 38.9).  Rows of
+// BK fp32 values, 16-byte chunks swizzled as the binary16 rows of as many.
+template <int R, int BK, int NW>
+struct SideA32D {
+    static constexpr int BYTES = R * BK * 4;
+    static constexpr int NINS = BYTES / 1024;
+    static constexpr int NLD = NINS / NW;
+    static_assert(NINS % NW == 0, "stage loads do not divide among the waves");
+    static constexpr int CPR = BK / 4;  // 16-byte chunks per LDS row
+    uint32_t off[NLD];
+    int kend[NLD];
+
+    __device__ __forceinline__ void init(int wave, int lane, int64_t ld, int mn0, int MN) {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            const int q = (wave * NLD + i) * 64 + lane;
+            const int row = q / CPR, c = (q % CPR) ^ swz_kc<CPR>(row);
+            off[i] = mn0 + row < MN ? (uint32_t)((int64_t)row * ld * 4 + c * 16) : kOob;
+            kend[i] = 4 * c + 4;
+        }
+    }
+    __device__ __forceinline__ void load(const float* tile, char* lds, int wave, int /*lane*/, int krem) const {
+        const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(tile);
+#pragma unroll
+        for (int i = 0; i < NLD; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t*)(lds + (wave * NLD + i) * 1024), 16,
+                                                     kend[i] <= krem ? off[i] : kOob, 0, 0, 0);
     }
 };
 
@@ -251,6 +295,17 @@ __device__ __forceinline__ half8_t read_frag(const char* lds, int rc0, int kk, i
     }
 }
 
+// The same fragment of an fp32 stage (SideA32D), converted.
+template <int BK>
+__device__ __forceinline__ half8_t read_frag_a32(const char* lds, int rc0, int kk, int lane) {
+    constexpr int CPR = BK / 4;
+    const int row = rc0 + (lane & 31), c = 4 * kk + 2 * (lane >> 5);
+    const char* p = lds + row * (CPR * 16);
+    const float4_t a = *reinterpret_cast<const float4_t*>(p + ((c ^ swz_kc<CPR>(row)) << 4));
+    const float4_t b = *reinterpret_cast<const float4_t*>(p + (((c + 1) ^ swz_kc<CPR>(row)) << 4));
+    return half8_clamped(a, b);
+}
+
 // Scheduling-group masks (LLVM AMDGPU sched_group_barrier).
 constexpr int kSgMfma = 0x008, kSgVmem = 0x010, kSgDsRead = 0x100;
 
@@ -265,17 +320,21 @@ constexpr int kSgMfma = 0x008, kSgVmem = 0x010, kSgDsRead = 0x100;
 // ZF: the stage's first k step starts each accumulator from zero (the
 // previous contents are dropped), as a product whose contraction begins here.
 template <bool A_KC, bool B_KC, int BM, int BN, int BK, int MI, int NI, int NV = 0, int EVERY = 1, int KN = BK / 16,
-          bool ZF = false>
+          bool ZF = false, bool A32 = false>
 __device__ __forceinline__ void mfma_stage(const char* la, const char* lb, int ar0, int bc0, int lane,
                                            float16_t (&acc)[MI][NI], int kk0 = 0) {
     constexpr int KS = KN;
-    constexpr int NR = (A_KC ? MI : 2 * MI) + (B_KC ? NI : 2 * NI);  // LDS reads per k step
-    constexpr int NM = MI * NI;                                      // MFMAs per k step
+    constexpr int NR = (A_KC && !A32 ? MI : 2 * MI) + (B_KC ? NI : 2 * NI);  // LDS reads per k step
+    constexpr int NM = MI * NI;                                              // MFMAs per k step
+    auto read_a = [&](int i, int kk) {
+        if constexpr (A32) return read_frag_a32<BK>(la, ar0 + 32 * i, kk, lane);
+        else return read_frag<A_KC, BM, BK>(la, ar0 + 32 * i, kk, lane);
+    };
     static_assert(NV <= KS * NM, "at most one load per MFMA");
     constexpr int EV = NV == 0 || NV * EVERY <= KS * NM ? EVERY : KS * NM / NV;  // spacing that fits
     half8_t af[2][MI], bf[2][NI];
 #pragma unroll
-    for (int i = 0; i < MI; ++i) af[0][i] = read_frag<A_KC, BM, BK>(la, ar0 + 32 * i, kk0, lane);
+    for (int i = 0; i < MI; ++i) af[0][i] = read_a(i, kk0);
 #pragma unroll
     for (int j = 0; j < NI; ++j) bf[0][j] = read_frag<B_KC, BN, BK>(lb, bc0 + 32 * j, kk0, lane);
 #pragma unroll
@@ -283,7 +342,7 @@ __device__ __forceinline__ void mfma_stage(const char* la, const char* lb, int a
         const int c = kk & 1, n = c ^ 1;
         if (kk + 1 < KS) {
 #pragma unroll
-            for (int i = 0; i < MI; ++i) af[n][i] = read_frag<A_KC, BM, BK>(la, ar0 + 32 * i, kk0 + kk + 1, lane);
+            for (int i = 0; i < MI; ++i) af[n][i] = read_a(i, kk0 + kk + 1);
 #pragma unroll
             for (int j = 0; j < NI; ++j) bf[n][j] = read_frag<B_KC, BN, BK>(lb, bc0 + 32 * j, kk0 + kk + 1, lane);
         }
@@ -370,23 +429,25 @@ __device__ __forceinline__ const T* gathered_tile(const GemmArgs& a, int m0, int
 #define VEDIC_A32_TILE(k) (HO ? gathered_tile<float>(args, m0, k) : A32f + (int64_t)m0 * args.lda + ((k) < K ? (k) : 0))
 #define VEDIC_B_TILE(k) \
     (B_KC ? B + (int64_t)n0 * args.ldb + ((k) < K ? (k) : 0) : B + (int64_t)((k) < K ? (k) : 0) * args.ldb + n0)
-// The loads of stage kt: A into (la) (an fp32 A into registers, committed
-// to (la) later), B into (lb).
+// The loads of stage kt: A into (la) (SideA32's into registers, committed to
+// (la) later), B into (lb).
 #define VEDIC_ISSUE(kt, la, lb)                                                          \
     do {                                                                                 \
         const int k_ = it.kb + (kt) * BK;                                                \
-        if constexpr (A32)                                                               \
+        if constexpr (A32R)                                                              \
             sa.load(VEDIC_A32_TILE(k_), it.ke - k_);                                     \
+        else if constexpr (A32)                                                          \
+            sa.load(VEDIC_A32_TILE(k_), (la), wave, lane, it.ke - k_);                   \
         else                                                                             \
             sa.load(VEDIC_A_TILE(k_), (la), wave, lane, it.ke - k_);                     \
         sb.load(VEDIC_B_TILE(k_), (lb), wave, lane, it.ke - k_);                         \
     } while (0)
-// The first ST - 1 stages of a work item; with an fp32 A each stage's A is
-// committed as soon as it has landed (its B may still be in flight).
+// The first ST - 1 stages of a work item; with an fp32 A in registers each
+// stage's A is committed as soon as it has landed (its B may still be in flight).
 #define VEDIC_PROLOGUE_STAGE(s_)                                                         \
     do {                                                                                 \
         VEDIC_ISSUE(s_, As[s_], Bs[s_]);                                                 \
-        if constexpr (A32) {                                                             \
+        if constexpr (A32R) {                                                            \
             wait_vmcnt<SB::NLD>();                                                       \
             sa.commit(As[s_], wave, lane);                                               \
         }                                                                                \
@@ -415,9 +476,10 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
     constexpr int WMN = WGM * WGN, NW = WMN * WGK, WM = BM / WGM, WN = BN / WGN, MI = WM / 32, NI = WN / 32;
     constexpr int KN = BK / 16 / WGK;
     static_assert(KN * WGK * 16 == BK, "the k steps of a stage divide among the wave groups");
-    constexpr bool A32 = OP == 3;
+    constexpr bool A32 = OP == 3, A32D = A32 && BM == 128, A32R = A32 && !A32D;  // an fp32 A: in LDS, in registers
     constexpr bool A_KC = OP != 2, B_KC = OP == 1;
-    using SA = std::conditional_t<A32, SideA32<BM, BK, NW>, Side<A_KC, BM, BK, NW>>;
+    using SA = std::conditional_t<A32R, SideA32<BM, BK, NW>,
+                                  std::conditional_t<A32D, SideA32D<BM, BK, NW>, Side<A_KC, BM, BK, NW>>>;
     using SB = Side<B_KC, BN, BK, NW>;
     constexpr int L = SA::NLD + SB::NLD;  // load instructions per wave per stage
     static_assert(ST >= 2 && ST <= 4, "2 to 4 LDS stages");
@@ -425,7 +487,7 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
     // 256 x 256 tiles: the stage's direct loads are spread one per MFMA instead
     // of issued together (2-3 % faster: fewer waves held at a full
     // texture-address queue); 128 x 128 tiles measured slower that way.
-    constexpr bool kInterleave = BM * BN >= 256 * 256 && WGK == 1 && HO == 0;
+    constexpr bool kInterleave = BM * BN >= 256 * 256 && WGK == 1 && HO == 0 && !A32;
     static_assert(HO == 0 || (WGK == 1 && (OP == 0 || OP == 3)), "gathered A: NN or AMP, one k group");
 
     // One LDS object per stage (A then B): reads of one stage provably do not
@@ -500,6 +562,24 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
             bias_pre[j] = pre_bias && col < args.N ? args.bias[col] : 0.0f;
         }
 
+        // Stage kt's MFMAs, and with HO the end of its head.
+        auto multiply = [&](const char* as, const char* bs, int kt) {
+            if constexpr (HO == 1) {
+                mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, true, A32D>(as, bs, wm * WM, wn * WN, lane, acc);
+                head_done();
+            } else {
+                mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, false, A32D>(as, bs, wm * WM, wn * WN, lane, acc,
+                                                                                 wk * KN);
+                if (HO == 2 && (kt + 1) % seg == 0) {
+                    head_done();
+#pragma unroll
+                    for (int i = 0; i < MI; ++i)
+#pragma unroll
+                        for (int j = 0; j < NI; ++j) acc[i][j] = float16_t{};
+                }
+            }
+        };
+
         // Uniform pipeline: every stage step waits for the same number of
         // loads and issues stage kt + ST - 1, which past the work item's
         // range loads zeros without touching memory; only the MFMAs are
@@ -512,7 +592,7 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
 #pragma unroll
             for (int s = 0; s < ST; ++s) {
                 const int kt = k0 + s;
-                if constexpr (A32) {
+                if constexpr (A32R) {
                     // A of stage kt was committed at the end of the previous
                     // step (everything issued before it has landed); B of
                     // stage kt is the newest batch when ST = 2
@@ -523,27 +603,11 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
                 }
                 stage_barrier();
                 const int sl = (s + ST - 1) % ST;
-                if constexpr (A32) {
+                if constexpr (A32R) {
                     // register loads, then the MFMAs, then the conversion into
                     // stage kt - 1's buffer, free since the barrier above
                     VEDIC_ISSUE(kt + ST - 1, As[sl], Bs[sl]);
-                    if (kt < nk) {
-                        if constexpr (HO == 1) {
-                            mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, true>(As[s], Bs[s], wm * WM, wn * WN,
-                                                                                      lane, acc);
-                            head_done();
-                        } else {
-                            mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN>(As[s], Bs[s], wm * WM, wn * WN, lane,
-                                                                                acc, wk * KN);
-                            if (HO == 2 && (kt + 1) % seg == 0) {
-                                head_done();
-#pragma unroll
-                                for (int i = 0; i < MI; ++i)
-#pragma unroll
-                                    for (int j = 0; j < NI; ++j) acc[i][j] = float16_t{};
-                            }
-                        }
-                    }
+                    if (kt < nk) multiply(As[s], Bs[s], kt);
                     wait_vmcnt<SB::NLD>();
                     sa.commit(As[sl], wave, lane);
                 } else if constexpr (kInterleave) {
@@ -556,23 +620,7 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
                     }
                 } else {
                     VEDIC_ISSUE(kt + ST - 1, As[sl], Bs[sl]);
-                    if (kt < nk) {
-                        if constexpr (HO == 1) {
-                            mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, true>(As[s], Bs[s], wm * WM, wn * WN,
-                                                                                      lane, acc);
-                            head_done();
-                        } else {
-                            mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN>(As[s], Bs[s], wm * WM, wn * WN, lane,
-                                                                                acc, wk * KN);
-                            if (HO == 2 && (kt + 1) % seg == 0) {
-                                head_done();
-#pragma unroll
-                                for (int i = 0; i < MI; ++i)
-#pragma unroll
-                                    for (int j = 0; j < NI; ++j) acc[i][j] = float16_t{};
-                            }
-                        }
-                    }
+                    if (kt < nk) multiply(As[s], Bs[s], kt);
                 }
             }
         }
@@ -635,9 +683,9 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
 #pragma unroll
         for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(bias_pre[j]));  // the bias has landed
         // The next work item's first stages go out before this epilogue
-        // (with an fp32 A after it: its staging registers would be live
+        // (with an fp32 A in registers after it: they would be live
         // across the epilogue).
-        if (!A32 && more) {
+        if (!A32R && more) {
             __syncthreads();  // every wave is done reading the stage buffers
             it = work_of<BM, BN, BK>(args, w, ntiles);
             m0 = it.m0;
@@ -659,7 +707,7 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
                 epilogue<KIND, true, MI, NI>(args, cp, acc, row0, col0, lane, pre_bias ? bias_pre : nullptr);
         }
         if (!more) break;
-        if constexpr (A32) {
+        if constexpr (A32R) {
             __syncthreads();
             it = work_of<BM, BN, BK>(args, w, ntiles);
             m0 = it.m0;
@@ -924,8 +972,8 @@ hipError_t launch_gemm_f16_direct_op(const GemmArgs& a, hipStream_t s) {
     }
     if constexpr (OP == 3) {
         // fp32 A: no 256 x 256 or 256 x 192 tiles (its staging registers do
-        // not fit beside their accumulators); 256 x 128 where the cost model
-        // picks one of those three, else 128 x 128
+        // not fit beside their accumulators); 256 x 128 where the cost model picks one of those three,
+        // else 128 x 128
         if (a.ksplit <= 1 && f16_tile_config(a.M, a.N, device_cu_count()) != 2)
             return launch_f16_kind<OP, CfgMid>(a, s);
         return launch_f16_kind<OP, CfgSmall>(a, s);

@@ -170,3 +170,27 @@ def test_amp_c_abi_entry_points():
                       A=x32.data_ptr(), lda=K, B=w16.data_ptr(), ldb=K, C=C.data_ptr(), ldc=N, alpha=1.0,
                       stream=s)
     assert lib.vedic_gemm(ctypes.byref(d)) == _lib.STATUS_BAD_DTYPE
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 520, 2048), (32, 520, 2048), (160, 513 // 8 * 8 + 8, 2056), (1531, 1024, 4096),
+                                   (129, 512, 2048), (129, 1024, 2040)])
+def test_long_contractions_around_the_cast_rule(M, N, K):
+    """More than 512 columns over 2048 or more steps are cast first, the rest
+    (and every call from a fixed scratch region) converted in the kernel: bit
+    for bit the cast + fp16 GEMM either way (past the decode kernel's rows)."""
+    import ctypes
+
+    from logos_amd import _lib, vedic
+
+    rng = np.random.default_rng(M + N + K)
+    x32, w32 = dev(normal(rng, (M, K))), dev(normal(rng, (K, N), std=0.05))
+    x32[0, 3], x32[M // 2, 1] = 1e6, float("-inf")
+    w16 = vedic.cast_fp32_to_fp16(w32)
+    C = vedic.amp_gemm(x32, w16)
+    if M > 32:
+        assert torch.equal(C, vedic.gemm_fp16_fp32out(vedic.cast_fp32_to_fp16(x32), w16))
+    C2 = torch.empty_like(C)
+    d = _lib.GemmDesc(op=0, in_dtype=_lib.DT_F32_F16, out_dtype=0, M=M, N=N, K=K, A=x32.data_ptr(), lda=K, B=w16.data_ptr(),
+                      ldb=N, C=C2.data_ptr(), ldc=N, alpha=1.0, stream=torch.cuda.current_stream().cuda_stream)
+    assert _lib.load().vedic_gemm_noalloc(ctypes.byref(d)) == 0
+    assert torch.equal(C, C2)
