@@ -1,5 +1,5 @@
 // vedic_flash_attn.hip -- fused attention forward for gfx950, fp32 in and out
-// (DH 64 on the bf16 matrix cores by exact splits, fa_item_split).
+// (on the bf16 matrix cores by exact splits, fa_item_split).
 //
 //   out = softmax(scale * Q . K^T + mask) . V          per head, Q/K/V/out [seq x DH]
 //
@@ -12,9 +12,10 @@
 //
 // Work item: one head, a group of 128 queries (four waves of 32) and a chunk
 // of keys.  The workgroup streams the chunk's keys through LDS in blocks of
-// 32 (K block and V block together, three stages in flight, direct
-// global -> LDS loads); every wave reuses each block for its own 32 queries.
-// Per block and wave:
+// 32 (K block and V block together); every wave reuses each block for its own
+// 32 queries.  Per block and wave, on the fp32 MFMA (fa_item, the repeat of
+// items that the split does not cover; two stages in flight by direct global ->
+// LDS loads):
 //   S^T [32 keys x 32 queries] = K_blk . Q^T     DH/2 x v_mfma_f32_32x32x2_f32
 //   running max / sum update, P = exp(S - max)   (lane l owns query l % 32)
 //   O^T [DH x 32 queries]     += V_blk^T . P^T   DH/2 x v_mfma_f32_32x32x2_f32
@@ -44,18 +45,18 @@ constexpr int fa_stage_bytes() {
     return 2 * kFaKeys * DH * 4;  // one stage: a K block, then a V block
 }
 
-// DH 128: two 32 KB stages, so two workgroups fit a CU (two waves per SIMD):
-// 8 heads x seq 8192 1360 -> 1327 us against three stages and one workgroup.
-#ifndef VEDIC_FA_ST128
-#define VEDIC_FA_ST128 2
-#endif
 #ifndef VEDIC_FA_WPE64
 #define VEDIC_FA_WPE64 3
 #endif
 #ifndef VEDIC_FA_WPE128
 #define VEDIC_FA_WPE128 2
 #endif
-// LDS stages in flight
+// LDS buffers of the blocks' bf16 parts
+template <int DH>
+constexpr int fa_buffers() {
+    return DH == 64 ? 2 : 1;
+}
+// LDS stages in flight of the fp32 repeat
 template <int DH>
 constexpr int fa_stages() {
     return 2;
@@ -275,14 +276,21 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
 }
 
 // The same work item on the bf16 matrix cores (vedic_split.hpp): K and V
-// blocks are split into three bf16 parts as they go from registers to LDS (two
-// buffers, one barrier per 32 keys, the block after next in flight), Q once per
-// item, P in registers.  Per block and wave DH / 16 x 6 MFMAs for S^T and
+// blocks are split into three bf16 parts as they go from registers to LDS, Q
+// once per item, P in registers.  Per block and wave DH / 16 x 6 MFMAs for S^T and
 // DH / 32 x 2 x 6 for O^T, 32 cycles each, against DH of 64 cycles on
 // v_mfma_f32_32x32x2_f32: 16 heads x seq 8192 causal 1213 -> 688-726 us, the
 // matrix pipe 62 % busy at 1.72 GHz, 6 VALU instructions (split, softmax) per
 // MFMA beside it.  scale log2(e) goes into Q before the split, so the
 // scores come out in base 2; V is scaled by 2^24 (vedic_split.hpp).
+//
+// DH 64: two LDS buffers, one barrier per 32 keys, the block after next in
+// flight.  DH 128: a block's parts are 48 KB, so two buffers would leave one
+// workgroup per CU, whose splits and softmax nothing overlaps; with one buffer
+// and two barriers two workgroups share a CU and one's matrix work covers the
+// other's split.  8 heads x seq 8192 causal: fp32 MFMA 1331 us, two buffers
+// 943, one 808; 8 x 1000: 51.9, 52.6, 42.2; one head x 8192: 203, 159, 126
+// (error against float64 6.3e-7 -> 5.3e-7).
 //
 // Returns whether the workgroup's results stand.  They do not if a sum is not
 // finite (an infinity or NaN among the operands, a value of 2^104 or more) or a
@@ -361,25 +369,39 @@ __device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char
             for (int d = 0; d < DH / 32; ++d) o[d] = mfma_split(fs_col<DH>(buf + KB, ad, d, j), pf, o[d]);
         }
     };
+    // Whether the wave's queries have a key in block kb (past the item's keys
+    // only for an odd count's last step of two buffers).
+    auto allowed = [&](int kb) {
+        const int key0 = w.k_lo + kb * kFaKeys;
+        return wave_live && kb < w.nkb && !(a.causal && key0 > q0 + 31) && !(a.sparse && !fa_sparse_any(a, key0, q0));
+    };
     // Step kb: block kb is in `cur`, block kb + 1 in registers.
     auto step = [&](const char* cur, char* nxt, int kb) {
-        const int key0 = w.k_lo + kb * kFaKeys;
         commit(nxt);
         load(kb + 2);
         ad.refresh();
-        // (past the item's keys only for an odd count's last step)
-        if (wave_live && kb < w.nkb && !(a.causal && key0 > q0 + 31) && !(a.sparse && !fa_sparse_any(a, key0, q0)))
-            compute(cur, key0);
+        if (allowed(kb)) compute(cur, w.k_lo + kb * kFaKeys);
         stage_barrier();
     };
 
     load(0);
-    commit(b0);
-    load(1);
-    stage_barrier();
-    for (int kb = 0; kb < w.nkb; kb += 2) {
-        step(b0, b1, kb);
-        step(b1, b0, kb + 1);
+    if constexpr (fa_buffers<DH>() == 1) {
+        for (int kb = 0; kb < w.nkb; ++kb) {
+            commit(b0);
+            load(kb + 1);
+            ad.refresh();
+            stage_barrier();
+            if (allowed(kb)) compute(b0, w.k_lo + kb * kFaKeys);
+            stage_barrier();  // every wave is done with the block before the next one overwrites it
+        }
+    } else {
+        commit(b0);
+        load(1);
+        stage_barrier();
+        for (int kb = 0; kb < w.nkb; kb += 2) {
+            step(b0, b1, kb);
+            step(b1, b0, kb + 1);
+        }
     }
 
     float probe = l_run * 0.0f;
@@ -395,25 +417,24 @@ __device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char
 // that take items from a counter until none is left: items run largest first,
 // so the tail of the key-split one-head case stays balanced.
 // DH 64: registers held to three waves per SIMD, the occupancy its 48 KB of
-// LDS allows (three workgroups per CU); DH 128: two (two 64 KB workgroups).
-template <int DH>
-constexpr bool fa_split() {
-    return DH == 64;
-}
+// LDS allows (three workgroups per CU); DH 128: two (two workgroups of 64 KB,
+// which the repeat's fp32 stages need).
 template <int DH>
 __device__ __forceinline__ void fa_run(const FlashArgs& a, int item, char* b0, char* b1) {
-    if constexpr (fa_split<DH>()) {
-        if (fa_item_split<DH>(a, item, b0, b1)) return;
-    }
+    if (fa_item_split<DH>(a, item, b0, b1)) return;
     fa_item<DH>(a, item, b0, b1);
 }
 template <int DH, bool QUEUE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DH == 64 ? VEDIC_FA_WPE64 : VEDIC_FA_WPE128)))
 flash_attn_kernel(FlashArgs a) {
-    // two LDS objects: reads of one stage provably do not alias writes of the other
-    constexpr int SB = fa_split<DH>() ? 2 * fs_block_bytes<DH>() : fa_stage_bytes<DH>();
+    // Two LDS objects: reads of one buffer provably do not alias writes of the
+    // other.  With one buffer its object holds the repeat's two fp32 stages.
+    constexpr bool two = fa_buffers<DH>() == 2;
+    constexpr int SB = two ? 2 * fs_block_bytes<DH>() : 2 * fa_stage_bytes<DH>();
+    static_assert(SB >= 2 * fs_block_bytes<DH>() && (!two || SB >= fa_stage_bytes<DH>()), "K and V parts; fp32 stages");
     __shared__ __attribute__((aligned(1024))) char b0[SB];
-    __shared__ __attribute__((aligned(1024))) char b1[SB];
+    __shared__ __attribute__((aligned(1024))) char bx[two ? SB : 16];
+    char* const b1 = two ? bx : b0 + fa_stage_bytes<DH>();
     __shared__ int next;
     if constexpr (!QUEUE) {
         fa_run<DH>(a, blockIdx.x, b0, b1);

@@ -11,7 +11,6 @@ namespace vedic {
 
 constexpr int kFaQ = 128;     // queries per work item (four waves x 32)
 constexpr int kFaKeys = 32;   // keys per LDS block
-constexpr int kFaStages = 3;  // LDS blocks in flight
 constexpr float kFaMasked = -1e30f;
 
 struct FlashArgs {

@@ -149,3 +149,36 @@ def test_backward_sparse_blocks(causal, window, stride):
     got = _backward(v, Q, K, V, dO, causal=bool(causal), shunyam=True, window=window, stride=stride)
     want = o.flash_attention_bwd_f64(Q, K, V, dO, 0.125, causal, 1, window, stride)
     assert o.grad_rel_err(got, want) <= fp32_tol(seq)
+
+
+@pytest.mark.parametrize("seq", [1, 31, 33, 129, 700])
+@pytest.mark.parametrize("causal,sparse", [(1, 0), (0, 0), (1, 1), (0, 1)])
+def test_forward_dh128(seq, causal, sparse):
+    """Head dimension 128 around the 32-key block and the 128-query group, one
+    head (its keys split over work items) and three: float64, and a head of
+    2^110 (repeated on the fp32 MFMA) beside two ordinary ones."""
+    v = vedic()
+    rng = np.random.default_rng(seq)
+    kw = dict(causal=bool(causal), shunyam=bool(sparse), window=40, stride=33)
+    for heads in (1, 3):
+        Q, K, V = ([normal(rng, (seq, 128)) for _ in range(heads)] for _ in range(3))
+        V[-1] = V[-1] * np.float32(2.0 ** 110)
+        outs = v.flash_attention_fwd_heads([dev(x) for x in Q], [dev(x) for x in K], [dev(x) for x in V], **kw)
+        for i in range(heads):
+            want = o.flash_attention_f64(Q[i], K[i], V[i], 128 ** -0.5, causal, sparse, 40, 33)
+            assert o.inf_rel_err(host(outs[i]), want) <= fp32_tol(128), (heads, i)
+
+
+@pytest.mark.parametrize("key", [0, 40, 299])
+def test_forward_dh128_nonfinite(key):
+    """An infinite V entry reaches the queries from its key on; the row groups
+    of 32 before it keep the finite call's values."""
+    v = vedic()
+    rng = np.random.default_rng(key)
+    Q, K, V = (normal(rng, (300, 128)) for _ in range(3))
+    clean = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V)))
+    V[key, 100] = np.inf
+    got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V)))
+    assert not np.any(np.isfinite(got[key:, 100]))
+    before = key // 32 * 32
+    assert np.all(np.abs(got[:before] - clean[:before]) <= fp32_tol(128) * np.abs(clean).max())
