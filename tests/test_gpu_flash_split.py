@@ -182,3 +182,20 @@ def test_forward_dh128_nonfinite(key):
     assert not np.any(np.isfinite(got[key:, 100]))
     before = key // 32 * 32
     assert np.all(np.abs(got[:before] - clean[:before]) <= fp32_tol(128) * np.abs(clean).max())
+
+
+@pytest.mark.parametrize("seq", [31, 33, 129, 300])
+@pytest.mark.parametrize("causal,sparse", [(1, 0), (0, 0), (1, 1), (0, 1)])
+@pytest.mark.parametrize("big", [False, True])
+def test_backward_dh128(seq, causal, sparse, big):
+    """Head dimension 128 around the 32-row block and the 128-row group; dO of
+    2^60 leaves the split's scaled sums (repeated on the fp32 MFMA)."""
+    v = vedic()
+    rng = np.random.default_rng(seq + 1000 * big)
+    kw = dict(causal=bool(causal), shunyam=bool(sparse), window=40, stride=33)
+    Q, K, V, dO = (normal(rng, (seq, 128)) for _ in range(4))
+    if big:
+        dO = dO * np.float32(2.0 ** 60)
+    got = _backward(v, Q, K, V, dO, **kw)
+    want = o.flash_attention_bwd_f64(Q, K, V, dO, 128 ** -0.5, causal, sparse, 40, 33)
+    assert o.grad_rel_err(got, want) <= fp32_tol(max(seq, 128))
