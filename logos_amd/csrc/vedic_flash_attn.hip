@@ -136,7 +136,7 @@ __device__ __forceinline__ void fa_store(const FlashArgs& a, const FaItem& w, co
 // One work item (`item` in decreasing size order) with the workgroup's two
 // LDS stages t0, t1.
 template <int DH>
-__device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, char* t1) {
+__device__ __forceinline__ void fa_item(const FlashArgs& a, int item, int tid, char* t0, char* t1) {
     constexpr int KB = kFaKeys * DH * 4;  // bytes of one K (or V) block
     constexpr int SB = fa_stage_bytes<DH>();
     constexpr int NLD = SB / 1024 / 4;    // 1 KiB direct loads per wave per stage
@@ -146,8 +146,8 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
     constexpr int FST = fa_stages<DH>();
     char* const stg[2] = {t0, t1};
 
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
 
     const FaItem w = fa_work<DH>(a, item);
     const int head = w.head, g = w.g, k_lo = w.k_lo, nkb = w.nkb;
@@ -279,10 +279,16 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
 // blocks are split into three bf16 parts as they go from registers to LDS, Q
 // once per item, P in registers.  Per block and wave DH / 16 x 6 MFMAs for S^T and
 // DH / 32 x 2 x 6 for O^T, 32 cycles each, against DH of 64 cycles on
-// v_mfma_f32_32x32x2_f32: 16 heads x seq 8192 causal 1213 -> 688-726 us, the
-// matrix pipe 62 % busy at 1.72 GHz, 6 VALU instructions (split, softmax) per
+// v_mfma_f32_32x32x2_f32: 16 heads x seq 8192 causal 1218 -> 757 us, the
+// matrix pipe 62 % busy at 1.72 GHz, 6.4 VALU instructions (split, softmax) per
 // MFMA beside it.  scale log2(e) goes into Q before the split, so the
-// scores come out in base 2; V is scaled by 2^24 (vedic_split.hpp).
+// scores come out in base 2.
+//
+// Factors against flushed parts (vedic_split.hpp).  Scores: 2^48 on Q, none on
+// K (no instruction per key); a part of K below 2^-126 that is lost then meets
+// |scale log2(e) Q| < 2^80, an error of a score below 2^-46.  The exponent
+// takes the 2^48 out in its subtraction (an fma).  Outputs, which have no scale
+// of their own: 2^24 on both P and V (16 heads x seq 8192 +1.6 %).
 //
 // DH 64: two LDS buffers, one barrier per 32 keys, the block after next in
 // flight.  DH 128: a block's parts are 48 KB, so two buffers would leave one
@@ -293,15 +299,14 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, char* t0, 
 // (error against float64 6.3e-7 -> 5.3e-7).
 //
 // Returns whether the workgroup's results stand.  They do not if a sum is not
-// finite (an infinity or NaN among the operands, a value of 2^104 or more) or a
-// row's largest score is below -1e28, which the fp32 kernel treats as masked;
-// then nothing has been written and the caller repeats the item with fa_item.
-// (Scores keep the fp32 error for |Q|, |K| < 2^76: values below 2^-126 flush.)
+// finite or a score is -inf: an infinity or NaN among the operands, a value past
+// the split's range (scale log2(e) Q of 2^80, V of 2^104), a score (base 2), a
+// partial sum of one, or an output past 2^80.  Then nothing has been written and
+// the caller repeats the item with fa_item.
 template <int DH>
-__device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char* b0, char* b1) {
+__device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, int tid, char* b0, char* b1) {
     constexpr int KB = fs_block_bytes<DH>();
     constexpr int NT = 256;
-    const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
     const FaItem w = fa_work<DH>(a, item);
@@ -312,12 +317,13 @@ __device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char
     const bool wave_live = q0 < a.seq;
 
     SplitFrag qf[DH / 16];
-    fs_load_rows<DH>(qf, a.q[w.head], query, a.seq, a.scale * 1.4426950408889634f, lane);
+    fs_load_rows<DH>(qf, a.q[w.head], query, a.seq, a.scale * (1.4426950408889634f * kSplitScale * kSplitScale), lane);
 
     float16_t o[DH / 32];
 #pragma unroll
     for (int d = 0; d < DH / 32; ++d) o[d] = float16_t{};
     float m_run = kFaMasked, l_run = 0.0f;
+    float low = 0.0f;  // the lowest score, or 0 (-inf would leave l and O finite)
 
     FsAddr<DH> ad(lane);
     FsStage<DH, NT> sk, sv;
@@ -335,16 +341,18 @@ __device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char
         float16_t s = float16_t{};
 #pragma unroll
         for (int j = 0; j < DH / 16; ++j) s = mfma_split(fs_row<DH>(buf, ad, j), qf[j], s);
-        // s[4 gg + r] is the score of key key0 + 8 gg + 4 h + r for this lane's query.
+        // s[4 gg + r] is 2^48 times the score of key key0 + 8 gg + 4 h + r for this lane's query.
+#pragma unroll
+        for (int i = 0; i < 16; ++i) low = fminf(low, s[i]);
         if (a.sparse || key0 + kFaKeys > a.seq || (a.causal && key0 + kFaKeys - 1 > q0)) {
 #pragma unroll
             for (int i = 0; i < 16; ++i)
-                s[i] = fa_allowed_score(a, s[i], key0 + 8 * (i >> 2) + 4 * h + (i & 3), query);
+                s[i] = fa_allowed(a, key0 + 8 * (i >> 2) + 4 * h + (i & 3), query) ? s[i] : -__builtin_inff();
         }
         float mx = s[0];
 #pragma unroll
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = fmaxf(mx, __shfl_xor(mx, 32)) * kSplitUnscale2;
         if (__any(mx > m_run)) {  // (a factor of 1 for every row otherwise)
             const float m_new = fmaxf(m_run, mx);
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -358,13 +366,13 @@ __device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char
         float ls = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            s[i] = __builtin_amdgcn_exp2f(s[i] - m_ref);
+            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], kSplitUnscale2, -m_ref));
             ls += s[i];
         }
         l_run += ls;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const SplitFrag pf = fs_acc(s, j);
+            const SplitFrag pf = fs_acc(s, j, kSplitScale);
 #pragma unroll
             for (int d = 0; d < DH / 32; ++d) o[d] = mfma_split(fs_col<DH>(buf + KB, ad, d, j), pf, o[d]);
         }
@@ -407,9 +415,8 @@ __device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char
     float probe = l_run * 0.0f;
 #pragma unroll
     for (int d = 0; d < DH / 32; ++d) probe = nonfinite_probe(o[d], probe);
-    const bool bad = probe != 0.0f || (m_run < -1e28f && m_run > kFaMasked);
-    if (__syncthreads_or(bad)) return false;
-    if (wave_live) fa_store<DH>(a, w, o, m_run, l_run, kSplitUnscale, wave, lane);
+    if (__syncthreads_or(probe != 0.0f || low == -__builtin_inff())) return false;
+    if (wave_live) fa_store<DH>(a, w, o, m_run, l_run, kSplitUnscale2, wave, lane);
     return true;
 }
 
@@ -421,8 +428,14 @@ __device__ __forceinline__ bool fa_item_split(const FlashArgs& a, int item, char
 // which the repeat's fp32 stages need).
 template <int DH>
 __device__ __forceinline__ void fa_run(const FlashArgs& a, int item, char* b0, char* b1) {
-    if (fa_item_split<DH>(a, item, b0, b1)) return;
-    fa_item<DH>(a, item, b0, b1);
+    // (The thread index is made opaque for each of the two, so that nothing they
+    // derive from it is computed before the loop over items and held in registers
+    // across it: 15 and 35 VGPRs spilled at DH 64 and 128 otherwise.)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    if (fa_item_split<DH>(a, item, tid & 255, b0, b1)) return;
+    asm volatile("" : "+v"(tid));
+    fa_item<DH>(a, item, tid & 255, b0, b1);
 }
 template <int DH, bool QUEUE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DH == 64 ? VEDIC_FA_WPE64 : VEDIC_FA_WPE128)))

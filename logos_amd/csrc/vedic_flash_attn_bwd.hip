@@ -480,7 +480,7 @@ __device__ __forceinline__ bool fb_dq_split(const FlashBwdArgs& a, int item, cha
         // dQ^T[d][q] += sum over keys K[key][d] dS^T[key][q]
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const SplitFrag sf = fs_acc(s, j);
+            const SplitFrag sf = fs_acc(s, j, 1.0f);
 #pragma unroll
             for (int d = 0; d < DH / 32; ++d) dq[d] = mfma_split(fs_col<DH>(buf, ad, d, j), sf, dq[d]);
         }
@@ -589,7 +589,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
         // dV^T[d][key] += sum over queries dO[q][d] P[q][key]
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const SplitFrag pf = fs_acc(s, j);
+            const SplitFrag pf = fs_acc(s, j, 1.0f);
 #pragma unroll
             for (int d = 0; d < DH / 32; ++d) dv[d] = mfma_split(fs_col<DH>(buf + KB, ad, d, j), pf, dv[d]);
         }
@@ -605,7 +605,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
         // dK^T[d][key] += sum over queries Q[q][d] dS[q][key]
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const SplitFrag sf = fs_acc(s, j);
+            const SplitFrag sf = fs_acc(s, j, 1.0f);
 #pragma unroll
             for (int d = 0; d < DH / 32; ++d) dk[d] = mfma_split(fs_col<DH>(buf, ad, d, j), sf, dk[d]);
         }

@@ -8,7 +8,7 @@
 namespace vedic {
 
 template <class Args>
-__device__ __forceinline__ float fa_allowed_score(const Args& a, float s, int key, int query) {
+__device__ __forceinline__ bool fa_allowed(const Args& a, int key, int query) {
     bool ok = key < a.seq;
     if (a.causal && key > query) ok = false;
     if (a.sparse) {
@@ -16,7 +16,11 @@ __device__ __forceinline__ float fa_allowed_score(const Args& a, float s, int ke
         const bool global = key % a.stride == 0;
         if (!in_window && !global) ok = false;
     }
-    return ok ? s : kFaMasked;
+    return ok;
+}
+template <class Args>
+__device__ __forceinline__ float fa_allowed_score(const Args& a, float s, int key, int query) {
+    return fa_allowed(a, key, query) ? s : kFaMasked;
 }
 
 // Whether the sparse mask (a.sparse set) leaves some of keys key0 .. key0 + 31

@@ -145,12 +145,12 @@ __device__ __forceinline__ void fs_load_rows(SplitFrag (&f)[DH / 16], const floa
     }
 }
 
-// The parts of accumulator registers 8 j .. 8 j + 7: the operand that meets
-// fs_col(.., j, ..).
-__device__ __forceinline__ SplitFrag fs_acc(const float16_t& s, int j) {
+// The parts of accumulator registers 8 j .. 8 j + 7, times `scale`: the operand
+// that meets fs_col(.., j, ..).
+__device__ __forceinline__ SplitFrag fs_acc(const float16_t& s, int j, float scale) {
     float w[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) w[e] = s[8 * j + e];
+    for (int e = 0; e < 8; ++e) w[e] = scale == 1.0f ? s[8 * j + e] : s[8 * j + e] * scale;
     return split8(w);
 }
 

@@ -68,6 +68,83 @@ def test_scales(heads, scales):
         assert np.abs(host(outs[i]) - want).max() <= fp32_tol(dh) * np.abs(want).max() + 4 * 2.0 ** -150
 
 
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("k", [60, 84, 96, 104, 110, 118, 125])
+def test_scores_from_far_apart_operands(dh, sign, k):
+    """Q of about 2^-k against K of about 2^k, and the other way round: scores of
+    order one, whose bits the parts of a tiny operand carry.  One head (its keys
+    split over work items) and three."""
+    v = vedic()
+    rng = np.random.default_rng(k + 1000 * dh + sign)
+    seq = 205
+    for heads in (1, 3):
+        Q, K, V = ([normal(rng, (seq, dh)) * np.float32(s) for _ in range(heads)]
+                   for s in (2.0 ** (-sign * k), 2.0 ** (sign * k), 1.0))
+        assert np.isfinite(Q).all() and np.isfinite(K).all()
+        outs = v.flash_attention_fwd_heads([dev(x) for x in Q], [dev(x) for x in K], [dev(x) for x in V])
+        for i in range(heads):
+            want = o.flash_attention_f64(Q[i], K[i], V[i], dh ** -0.5, 1, 0, 0, 1)
+            # (a score of up to 4: 4 sqrt(dh) roundings of its size)
+            assert o.inf_rel_err(host(outs[i]), want) <= 16 * np.sqrt(dh) * o.U32, (heads, i)
+
+
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("e", [90, 84, 78, 50])
+def test_scores_past_the_split(dh, e):
+    """Scores of size 2^e, some rows all negative: past 2^80 the scaled scores
+    are infinite and the item is repeated, also where every one is -inf."""
+    v = vedic()
+    rng = np.random.default_rng(e + dh)
+    seq = 150
+    K, V = np.abs(normal(rng, (seq, dh))), normal(rng, (seq, dh))
+    Q = np.abs(normal(rng, (seq, dh))) * np.float32(2.0 ** e)
+    Q[::2] = -Q[::2]
+    got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V)))
+    # (scores this far apart leave one key per row; two whose scores lie within
+    # the rounding of their sum would be a tie that binary32 cannot decide)
+    s = (Q.astype(np.float64) @ K.astype(np.float64).T) * dh ** -0.5
+    s[np.triu_indices(seq, 1)] = -np.inf
+    top = np.sort(s, 1)[:, ::-1]
+    clear = np.r_[True, top[1:, 0] - top[1:, 1] > fp32_tol(dh) * np.abs(top[1:, 1])]
+    assert clear.sum() > 140
+    want = o.flash_attention_f64(Q, K, V, dh ** -0.5, 1, 0, 0, 1)
+    assert np.abs(got[clear] - want[clear]).max() <= fp32_tol(dh) * np.abs(want).max()
+
+
+def test_infinite_score_that_cancels():
+    """Partial sums of a score that leave the split's range and come back: -2^100
+    from one group of 16 values, +2^100 from the next, the rest of order one."""
+    v = vedic()
+    rng = np.random.default_rng(31)
+    seq, dh = 70, 64
+    Q, K, V = (normal(rng, (seq, dh)) for _ in range(3))
+    Q[:, 3] = Q[:, 20] = 2.0 ** 50
+    K[:, 3], K[:, 20] = -2.0 ** 50, 2.0 ** 50
+    Q[:, 4:20] = Q[:, :3] = Q[:, 21:] = 0  # (what else a partial sum of 2^100 holds would be rounded away)
+    got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V)))
+    want = o.flash_attention_f64(Q, K, V, 0.125, 1, 0, 0, 1)
+    assert o.inf_rel_err(got, want) <= fp32_tol(dh)
+
+
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("t", [60, 105, 112, 118, 124])
+def test_tiny_probabilities(dh, t):
+    """A key of probability 2^-t that holds the only values: its outputs keep
+    the accuracy that the score's rounding leaves the probability."""
+    v = vedic()
+    rng = np.random.default_rng(t)
+    seq = 100
+    Q, K, V = np.zeros((seq, dh), np.float32), np.zeros((seq, dh), np.float32), np.zeros((seq, dh), np.float32)
+    Q[:, 0] = 1 + 0.01 * rng.random(seq)
+    K[7, 0] = -t * np.log(2.0) * dh ** 0.5
+    V[7] = normal(rng, (dh,)) * np.float32(2.0 ** 76)
+    got = host(v.flash_attention_fwd(dev(Q), dev(K), dev(V), causal=False)).astype(np.float64)
+    want = o.flash_attention_f64(Q, K, V, dh ** -0.5, 0, 0, 0, 1)
+    # the score t: 4 roundings (scale, Q, product, exponent) of t u each, and the sums of the row
+    assert np.abs(got - want).max() <= (4 * t + 4 * np.sqrt(seq)) * o.U32 * np.abs(want).max()
+
+
 def test_scores_far_below_zero():
     """Rows whose every score is about -2^101: below -1e29 the reference counts
     a score as masked."""
