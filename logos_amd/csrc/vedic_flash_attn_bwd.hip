@@ -379,25 +379,25 @@ __device__ __forceinline__ void fb_dkdv_item(const FlashBwdArgs& a, int item, ch
 // Both passes with every operand split exactly into three bf16 parts
 // (vedic_split.hpp): the streamed blocks once per workgroup on their way into
 // LDS (two buffers, one barrier per 32 rows), the resident rows once per item,
-// P and dS in registers.  K, V and dO carry the factor 2^24 of the split, Q
-// (dK/dV pass) too; scale log2(e) 2^-24 goes into the other side of the score
-// product, so scores come out in base 2; dP, D and dS carry 2^48 and the
-// accumulators 2^72 (dV: P is not scaled, 2^24).
+// P and dS in registers.  Every operand carries the split's factor 2^24, scale
+// log2(e) with the resident side of the score product: scores come out in base
+// 2 times 2^48, which the exponent takes out in its subtraction (an fma).  dP, D
+// and dS carry 2^48, the accumulators 2^72 (dV: 2^48).
 //
 // Bound: the matrix cores, 72 and 96 MFMAs of 32 cycles per 32 x 32 block
-// (fp32: 96 and 128 of 64).  16 heads x seq 8192 causal 4253 -> 2303 us per
+// (fp32: 96 and 128 of 64).  16 heads x seq 8192 causal 4241 -> 2307 us per
 // backward (error against float64 2.2e-6 -> 1.6e-6): 61 and 60 % of the matrix
-// pipe busy at two waves per SIMD (231 and 254 registers), at the 1.83 GHz the
+// pipe busy at two waves per SIMD (246 and 254 registers), at the 1.83 GHz the
 // chip holds under this load.
 // DH 128 (144 and 192 MFMAs per block): one wave per SIMD, 96 and 97 KB of LDS,
 // no spill; K, V, dK and dV of 32 keys fit beside two score blocks, so that S is
-// computed once for dK and dV.  8 heads x seq 8192 causal 5486 -> 2511 us per
-// backward (2.2e-6 -> 1.6e-6), 8 x 1000 665 -> 309, DH 80 (padded) x 2500
+// computed once for dK and dV.  8 heads x seq 8192 causal 5461 -> 2554 us per
+// backward (2.2e-6 -> 1.6e-6), 8 x 1000 676 -> 320, DH 80 (padded) x 2500
 // not causal 1655 -> 785.
 //
-// As in the forward, an item whose sums are not finite is repeated on the
-// fp32 MFMA (with nothing written before but the same lse2 and D).  Scores
-// keep the fp32 error for |Q|, |K| < 2^76.
+// As in the forward, an item is repeated on the fp32 MFMA (with nothing written
+// before but the same lse2 and D) if a sum is not finite or a score is -inf (its
+// probability of 0 would leave the sums finite).
 constexpr float kFbScale2 = kSplitScale * kSplitScale;  // 2^48
 constexpr float kFbUnscale3 = kSplitUnscale2 * kSplitUnscale;  // 2^-72
 
@@ -415,7 +415,7 @@ __device__ __forceinline__ bool fb_dq_split(const FlashBwdArgs& a, int item, cha
     const bool live = q0 < a.seq;
 
     SplitFrag qf[DH / 16], df[DH / 16];
-    fs_load_rows<DH>(qf, a.q[head], query, a.seq, a.scale * (1.4426950408889634f * kSplitUnscale), lane);
+    fs_load_rows<DH>(qf, a.q[head], query, a.seq, a.scale * (1.4426950408889634f * kSplitScale), lane);
     float dsum = 0.0f;
     {
         const __amdgpu_buffer_rsrc_t rd = buffer_rsrc(a.dout[head]), ro = buffer_rsrc(a.o[head]);
@@ -446,6 +446,7 @@ __device__ __forceinline__ bool fb_dq_split(const FlashBwdArgs& a, int item, cha
         st[1] = D;
     }
     const float D2 = D * kFbScale2;
+    float low = 0.0f;  // the lowest score, or 0
 
     float16_t dq[DH / 32];
 #pragma unroll
@@ -469,7 +470,10 @@ __device__ __forceinline__ bool fb_dq_split(const FlashBwdArgs& a, int item, cha
         for (int j = 0; j < DH / 16; ++j) dp = mfma_split(fs_row<DH>(buf + KB, ad, j), df[j], dp);
         // s[4 gg + r]: key key0 + 8 gg + 4 h + r of this lane's query
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(s[i] - lse2);
+        for (int i = 0; i < 16; ++i) {
+            low = fminf(low, s[i]);
+            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], kSplitUnscale2, -lse2));
+        }
         if (a.sparse || key0 + 32 > a.seq || (a.causal && key0 + 31 > q0)) {
 #pragma unroll
             for (int i = 0; i < 16; ++i)
@@ -506,9 +510,8 @@ __device__ __forceinline__ bool fb_dq_split(const FlashBwdArgs& a, int item, cha
     float probe = 0.0f;
 #pragma unroll
     for (int d = 0; d < DH / 32; ++d) probe = nonfinite_probe(dq[d], probe);
-    if (__syncthreads_or(probe != 0.0f)) return false;
+    if (__syncthreads_or(probe != 0.0f || low == -__builtin_inff())) return false;
     if (!live || query >= a.seq) return true;
-    const float f = a.scale * kFbUnscale3;
     float* row = a.dq[head] + (int64_t)query * DH;
 #pragma unroll
     for (int d = 0; d < DH / 32; ++d)
@@ -516,7 +519,7 @@ __device__ __forceinline__ bool fb_dq_split(const FlashBwdArgs& a, int item, cha
         for (int gg = 0; gg < 4; ++gg) {
             float4_t v;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = dq[d][4 * gg + r] * f;
+            for (int r = 0; r < 4; ++r) v[r] = dq[d][4 * gg + r] * kFbUnscale3 * a.scale;
             store16_hold(row + 32 * d + 8 * gg + 4 * h, v);
         }
     return true;
@@ -543,7 +546,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
     const bool live = k0 < a.seq;
 
     SplitFrag kf[DH / 16], vf[DH / 16];
-    fs_load_rows<DH>(kf, a.k[head], key, a.seq, a.scale * (1.4426950408889634f * kSplitUnscale), lane);
+    fs_load_rows<DH>(kf, a.k[head], key, a.seq, a.scale * (1.4426950408889634f * kSplitScale), lane);
     fs_load_rows<DH>(vf, a.v[head], key, a.seq, kSplitScale, lane);
     const float* stats = a.delta + (int64_t)head * a.seq * 2;
 
@@ -555,7 +558,8 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
     }
     FsAddr<DH> ad(lane);
     FsStage<DH, NT> sq, sd;
-    float st = 0.0f;  // threads 0 .. 63: the block's lse2 and D, interleaved
+    float st = 0.0f;   // threads 0 .. 63: the block's lse2 and D, interleaved
+    float low = 0.0f;  // the lowest score, or 0
     auto load = [&](int qb) {
         const int q0 = (qstart + qb) * 32, rows = qb < nqb ? a.seq - q0 : 0;
         sq.load(a.q[head], q0, rows, tid);
@@ -576,10 +580,17 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
         for (int j = 0; j < DH / 16; ++j) s = mfma_split(fs_row<DH>(buf, ad, j), kf[j], s);
         // s[4 gg + r]: query qb0 + 8 gg + 4 h + r against this lane's key
 #pragma unroll
+        for (int i = 0; i < 16; ++i) low = fminf(low, s[i]);
+        if constexpr (DH == 64) {  // (no register is left to carry it: NaN in dV from here on if a score is -inf)
+            dv[0][0] = __builtin_fmaf(low, 0.0f, dv[0][0]);
+            low = 0.0f;
+        }
+#pragma unroll
         for (int gg = 0; gg < 4; ++gg) {
             const float4_t lse2 = *reinterpret_cast<const float4_t*>(sl + 32 * gg);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s[4 * gg + r] = __builtin_amdgcn_exp2f(s[4 * gg + r] - lse2[r]);
+            for (int r = 0; r < 4; ++r)
+                s[4 * gg + r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * gg + r], kSplitUnscale2, -lse2[r]));
         }
         if (a.sparse || (a.causal && qb0 < k0 + 31)) {
 #pragma unroll
@@ -589,7 +600,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
         // dV^T[d][key] += sum over queries dO[q][d] P[q][key]
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const SplitFrag pf = fs_acc(s, j, 1.0f);
+            const SplitFrag pf = fs_acc(s, j, kSplitScale);
 #pragma unroll
             for (int d = 0; d < DH / 32; ++d) dv[d] = mfma_split(fs_col<DH>(buf + KB, ad, d, j), pf, dv[d]);
         }
@@ -631,9 +642,8 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
 #pragma unroll
     for (int d = 0; d < DH / 32; ++d) probe = nonfinite_probe(dk[d], nonfinite_probe(dv[d], probe));
     // (keys past seq are not stored: their sums may be anything)
-    if (__syncthreads_or(key < a.seq && probe != 0.0f)) return false;
+    if (__syncthreads_or(key < a.seq && (probe != 0.0f || low == -__builtin_inff()))) return false;
     if (!live || key >= a.seq) return true;
-    const float f = a.scale * kFbUnscale3;
     float* vrow = a.dv[head] + (int64_t)key * DH;
     float* krow = a.dk[head] + (int64_t)key * DH;
 #pragma unroll
@@ -643,8 +653,8 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
             float4_t v, w;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                v[r] = dv[d][4 * gg + r] * kSplitUnscale;
-                w[r] = dk[d][4 * gg + r] * f;
+                v[r] = dv[d][4 * gg + r] * kSplitUnscale2;
+                w[r] = dk[d][4 * gg + r] * kFbUnscale3 * a.scale;
             }
             store16_hold(vrow + 32 * d + 8 * gg + 4 * h, v);
             store16_hold(krow + 32 * d + 8 * gg + 4 * h, w);

@@ -198,6 +198,45 @@ def test_backward_scales(scales):
         assert np.abs(g - w).max() <= fp32_tol(seq) * np.abs(w).max(), name
 
 
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("grad", [-20, -60])
+@pytest.mark.parametrize("k", [60, 84, 90, 96, 104, 110, 118, 125])
+def test_backward_from_far_apart_operands(dh, sign, grad, k):
+    """Q of about 2^-k against K of about 2^k, and the other way round: scores of
+    order one, gradients small enough that no sum leaves the split's range."""
+    v = vedic()
+    rng = np.random.default_rng(k + 1000 * dh + sign)
+    seq = 205
+    Q, K, V, dO = (normal(rng, (seq, dh)) * np.float32(s) for s in (2.0 ** (-sign * k), 2.0 ** (sign * k), 1.0, 2.0 ** grad))
+    got = _backward(v, Q, K, V, dO)
+    want = o.flash_attention_bwd_f64(Q, K, V, dO, dh ** -0.5)
+    for g, w, name in zip(got, want, ("dQ", "dK", "dV")):
+        # (scores of up to 4: 4 sqrt(dh) roundings of their size, then sums of seq
+        # terms; subnormal sums are rounded to 2^-149 at every term)
+        bound = (16 * np.sqrt(dh) + 4 * np.sqrt(seq)) * o.U32 * np.abs(w).max() + seq * 2.0 ** -149
+        assert np.abs(g - w).max() <= bound, name
+
+
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("t", [60, 100, 105, 112, 118])
+def test_backward_tiny_probabilities(dh, t):
+    """dV of a key that every query gives a probability of about 2^-t / 100."""
+    v = vedic()
+    rng = np.random.default_rng(t)
+    seq = 100
+    Q, K = np.zeros((seq, dh), np.float32), np.zeros((seq, dh), np.float32)
+    V, dO = normal(rng, (seq, dh)), normal(rng, (seq, dh))
+    Q[:, 0] = 1 + 0.01 * rng.random(seq)
+    K[7, 0] = -t * np.log(2.0) * dh ** 0.5
+    got = _backward(v, Q, K, V, dO, causal=False)[2][7].astype(np.float64)
+    want = o.flash_attention_bwd_f64(Q, K, V, dO, dh ** -0.5, 0)[2][7]
+    # the score t: 4 roundings (scale, K, product, exponent) of t u each on every
+    # term, and the sum of the seq terms
+    size = (np.abs(dO).astype(np.float64).sum(0) * 2.0 ** -t / seq).max()
+    assert np.abs(got - want).max() <= (4 * t + 4 * np.sqrt(seq)) * o.U32 * size
+
+
 def test_backward_nonfinite():
     """A NaN in one dO row reaches every dK, dV row it attends to and its own
     dQ row; the other queries keep their finite dQ and the keys past its
