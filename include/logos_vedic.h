@@ -37,8 +37,18 @@
  * reused by every later call on that stream (their work runs in stream
  * order), and held until the process ends or vedic_workspace_release(stream).
  * Host threads may share a stream: a call holds the block from its first
- * request until its last kernel is enqueued.  Results never depend on the
- * split or on timing: slices are added in a fixed order.
+ * request until its last kernel is enqueued.  Results never depend on timing:
+ * slices are added in a fixed order.
+ *
+ * Stream capture: nothing is allocated during one.  The first captured call
+ * that needs temporaries takes over the block that an earlier call left on the
+ * stream (run the largest call once before the capture, and let it finish
+ * before the graph is launched); the graph keeps it until
+ * vedic_workspace_release(stream), to be called after the graph's last launch.
+ * Without one, products and attention run unsplit and AMP products convert in
+ * the kernel where they can, and a call that cannot do without memory returns
+ * VEDIC_STATUS_HIP_ERROR (hipErrorStreamCaptureUnsupported) and records
+ * nothing.  vedic_gemm_noalloc never needs the block.
  *
  * Errors follow the reference's conventions: shape errors are
  * VEDIC_STATUS_BAD_DIM (the reference throws std::invalid_argument,

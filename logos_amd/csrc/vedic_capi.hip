@@ -13,6 +13,7 @@
 #include <mutex>
 #include <tuple>
 #include <utility>
+#include <vector>
 
 #include "../../include/logos_vedic.h"
 #include "vedic_flash_attn.hpp"
@@ -79,10 +80,49 @@ static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; 
 // the same memory.  Workspaces nested in one call (same thread) carve after
 // the outer one's pieces.  The memory is held until the process ends or
 // vedic_workspace_release is called for the stream.
+//
+// Stream capture.  A graph is replayed at any time and on any stream, so what
+// a captured call writes to must be no other call's memory, and nothing is
+// allocated while capturing (memory from hipMallocAsync nodes of a graph
+// faulted on replay here).  The first captured call that needs temporaries
+// therefore takes over the block that earlier calls left on the stream: it
+// serves the calls of that capture (in stream order, one after the other) and
+// is held until vedic_workspace_release, while the stream's later calls get a
+// new one.
+struct ArenaBlock {
+    char* base = nullptr;
+    size_t cap = 0, used = 0;
+    unsigned long long capture = 0;  // of a block that a capture took over: its id
+};
 struct StreamArena {
     std::recursive_mutex mu;
-    char* base = nullptr;
-    size_t cap = 0, used = 0, want = 0;
+    ArenaBlock main;
+    size_t want = 0;
+    std::vector<ArenaBlock*> held;  // blocks of captures
+
+    // Makes the block as large as the largest call so far (the old one is freed
+    // after the work queued on it).
+    void grow(hipStream_t s) {
+        if (main.used != 0 || want <= main.cap) return;
+        if (main.base) (void)hipFreeAsync(main.base, s);
+        main = ArenaBlock();
+        if (hipMallocAsync(reinterpret_cast<void**>(&main.base), want, s) == hipSuccess)
+            main.cap = want;
+        else
+            main.base = nullptr;
+    }
+    // The block of the capture `id`; null if none was there to take over.
+    ArenaBlock* captured_block(unsigned long long id) {
+        for (ArenaBlock* b : held)
+            if (b->capture == id) return b;
+        if (main.base == nullptr || main.used != 0) return nullptr;
+        ArenaBlock* b = new ArenaBlock(main);
+        b->capture = id;
+        held.push_back(b);
+        if (want < main.cap) want = main.cap;
+        main = ArenaBlock();
+        return b;
+    }
 };
 
 // Arenas and work-queue counters are kept per (device, stream handle, owner).
@@ -147,18 +187,22 @@ static hipError_t flash_queue_release(hipStream_t s) {
 
 // One call's temporaries: pieces carved in order from the stream's arena (a
 // piece that does not fit comes from the stream-ordered pool, and the arena
-// grows to fit the whole call at the next call's first request).  Bound to a
-// fixed region instead (the allocation-free entry point), pieces are carved
-// from it and nothing is allocated or freed; a request past its end sets
-// `overflow` and fails, and the call reports VEDIC_STATUS_TOO_LARGE.
+// grows to fit the whole call when it ends; in a captured call it is an
+// error).  Bound to a fixed region instead (the allocation-free entry point),
+// pieces are carved from it and nothing is allocated or freed; a request past
+// its end sets `overflow` and fails, and the call reports VEDIC_STATUS_TOO_LARGE.
 struct Workspace {
     hipStream_t s = nullptr;
     char* region = nullptr;  // non-null: carve from [region, region + cap)
     size_t cap = 0, used = 0;
     bool overflow = false;
     StreamArena* arena = nullptr;  // locked while this workspace is alive
-    size_t mark = 0;               // the arena's fill when this workspace took it
+    ArenaBlock* block = nullptr;   // the arena's block that serves this call
+    size_t mark = 0;               // its fill when this workspace took it
+    size_t asked = 0;              // all pieces of this call so far
     void* extra[8] = {};           // pieces from the pool (did not fit the arena)
+    int captured = -1;             // whether the stream is being captured (-1: not asked yet)
+    unsigned long long capture_id = 0;
 
     Workspace() = default;
     Workspace(const Workspace&) = delete;
@@ -166,16 +210,33 @@ struct Workspace {
     ~Workspace() {
         for (void* p : extra)
             if (p) (void)hipFreeAsync(p, s);
+        if (block) block->used = mark;
         if (arena) {
-            arena->used = mark;
+            if (!capturing()) arena->grow(s);  // so that one call is enough before a capture
             arena->mu.unlock();
         }
     }
 
     bool fixed() const { return region != nullptr; }
+    // (the null stream cannot be captured)
+    bool capturing() {
+        if (captured < 0) {
+            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+            captured = s != nullptr && hipStreamGetCaptureInfo(s, &st, &capture_id) == hipSuccess &&
+                       st != hipStreamCaptureStatusNone;
+        }
+        return captured != 0;
+    }
+    static size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    // Whether a captured call can have `bytes` more (any other call can).
+    bool room(size_t bytes) {
+        if (fixed() || !capturing()) return true;
+        open();
+        return block != nullptr && rounded(bytes) <= block->cap - block->used;
+    }
     template <typename T>
     hipError_t get(T** p, size_t bytes) {
-        const size_t take = (bytes + 255) / 256 * 256;
+        const size_t take = rounded(bytes);
         if (fixed()) {
             if (take > cap - used) {
                 overflow = true;
@@ -185,34 +246,15 @@ struct Workspace {
             used += take;
             return hipSuccess;
         }
-        if (!arena) {
-            StreamArena* a = arena_of(s);
-            a->mu.lock();
-            arena = a;
-            mark = a->used;
-            // (not inside a stream capture: the block would belong to the graph;
-            // its pieces come from the pool, as nodes of the graph)
-            hipStreamCaptureStatus cap_status = hipStreamCaptureStatusNone;
-            if (a->used == 0 && a->want > a->cap &&
-                (s == nullptr || hipStreamIsCapturing(s, &cap_status) != hipSuccess ||
-                 cap_status == hipStreamCaptureStatusNone)) {
-                // grow (the old block is freed after the work queued on it)
-                if (a->base) (void)hipFreeAsync(a->base, s);
-                a->base = nullptr;
-                a->cap = 0;
-                if (hipMallocAsync(reinterpret_cast<void**>(&a->base), a->want, s) == hipSuccess)
-                    a->cap = a->want;
-                else
-                    a->base = nullptr;
-            }
-        }
-        StreamArena* a = arena;
-        if (take <= a->cap - a->used) {
-            *p = reinterpret_cast<T*>(a->base + a->used);
-            a->used += take;
+        open();
+        asked += take;
+        if (block && take <= block->cap - block->used) {
+            *p = reinterpret_cast<T*>(block->base + block->used);
+            block->used += take;
             return hipSuccess;
         }
-        if (a->used + take > a->want) a->want = a->used + take;
+        if (capturing()) return hipErrorStreamCaptureUnsupported;
+        if (mark + asked > arena->want) arena->want = mark + asked;
         for (void*& slot : extra)
             if (!slot) {
                 const hipError_t e = hipMallocAsync(reinterpret_cast<void**>(p), bytes, s);
@@ -231,6 +273,22 @@ struct Workspace {
                 return hipFreeAsync(p, s);
             }
         return hipSuccess;
+    }
+
+private:
+    // Takes the stream's arena for this call.
+    void open() {
+        if (arena) return;
+        StreamArena* a = arena_of(s);
+        a->mu.lock();
+        arena = a;
+        if (capturing()) {
+            block = a->captured_block(capture_id);
+        } else {
+            a->grow(s);
+            block = &a->main;
+        }
+        if (block) mark = block->used;
     }
 };
 
@@ -704,24 +762,28 @@ static int gemm_impl(const vedic_gemm_desc_t* d, float* const* heads, int nheads
     const bool f16 = d->in_dtype != VEDIC_DT_F32;
     // (an fp32 A's tile rows are twice as long in bytes)
     const bool direct = vec && d->lda < (amp ? kMaxLd / 2 : kMaxLd) && d->ldb < kMaxLd;
+    hipStream_t s = static_cast<hipStream_t>(d->stream);
+    Workspace pool;
+    pool.s = s;
+    Workspace& ws = wsp ? *wsp : pool;
     // (a caller's fixed scratch region is asked for a copy of A only where it
-    // must: the bits are the same)
-    if (amp && (!direct || (wsp ? d->N > kAmpInKernelMaxN : amp_cast_first(d->M, d->N, d->K))))
-        return amp_via_cast(d, heads, nheads, head_cols, handoff, wsp);
+    // must, and a captured call does without where it can: the bits are the same)
+    if (amp && (!direct || (wsp ? d->N > kAmpInKernelMaxN : amp_cast_first(d->M, d->N, d->K))) &&
+        (!direct || ws.room(sizeof(_Float16) * (size_t)d->M * d->K)))
+        return amp_via_cast(d, heads, nheads, head_cols, handoff, &ws);
     // scattered C needs the kernels with a plain or bias epilogue kind
     if (scatter && !direct) return VEDIC_STATUS_BAD_LD;
     const bool skinny = direct && !amp && d->op == VEDIC_OP_NN && d->M <= 32;
     const int kop = amp ? kOpAmp : d->op;  // the fp16 kernels' op
     // (fp32 products that the wave-split 32 x 64 tiles fill are not split over workgroups)
     const bool wave_split = !f16 && direct && d->op != VEDIC_OP_TN && f32_wave_split(d->M, d->N, device_cu_count());
-    const int ks = skinny || scatter || wave_split || (f16 && !direct)
-                       ? 1
-                       : choose_ksplit(d->M, d->N, d->K, device_cu_count(), f16);
-
-    hipStream_t s = static_cast<hipStream_t>(d->stream);
-    Workspace pool;
-    pool.s = s;
-    Workspace& ws = wsp ? *wsp : pool;
+    int ks = skinny || scatter || wave_split || (f16 && !direct)
+                 ? 1
+                 : choose_ksplit(d->M, d->N, d->K, device_cu_count(), f16);
+    // (in a capture without memory for the slices the product runs unsplit)
+    if (ks > 1 && !ws.room(sizeof(float) * (size_t)d->M * d->N * ks +
+                           (d->colsum ? Workspace::rounded(sizeof(float) * colsum_matrix_floats(d->M, d->N)) : 0)))
+        ks = 1;
     hipError_t e = hipSuccess;
     // Column sums: the fused epilogue writes one partial per 32-row block and
     // column, added afterwards in a fixed order.  A split product sums the
@@ -833,9 +895,7 @@ __global__ void cast_rows8_f16_kernel(const float* __restrict__ src, int64_t lds
 static int amp_via_cast(const vedic_gemm_desc_t* d, float* const* heads, int nheads, int head_cols,
                         ColsumHandoff* handoff, Workspace* wsp) {
     hipStream_t s = static_cast<hipStream_t>(d->stream);
-    Workspace pool;
-    pool.s = s;
-    Workspace& ws = wsp ? *wsp : pool;
+    Workspace& ws = *wsp;
     _Float16* a16 = nullptr;
     hipError_t e = ws.get(&a16, sizeof(_Float16) * (size_t)d->M * d->K);
     if (e != hipSuccess) return ws.overflow ? VEDIC_STATUS_TOO_LARGE : hip_status(e);
@@ -907,9 +967,14 @@ extern "C" int vedic_workspace_release(void* stream) {
     StreamArena* a = arena_of(s);
     std::lock_guard<std::recursive_mutex> lk(a->mu);
     hipError_t e = hipSuccess;
-    if (a->base) e = hipFreeAsync(a->base, s);
-    a->base = nullptr;
-    a->cap = 0;
+    if (a->main.base) e = hipFreeAsync(a->main.base, s);
+    a->main = ArenaBlock();
+    for (ArenaBlock* b : a->held) {  // (their graphs are gone, or not replayed again)
+        const hipError_t f = hipFreeAsync(b->base, s);
+        if (e == hipSuccess) e = f;
+        delete b;
+    }
+    a->held.clear();
     a->want = 0;
     const hipError_t f = flash_queue_release(s);
     return hip_status(e != hipSuccess ? e : f);
@@ -1991,12 +2056,26 @@ static int flash_launch(FlashArgs& a, int dh, Workspace& wsf) {
     // Workspace: the chunk partials.  The split items go to a grid of
     // resident workgroups (LDS allows three per CU at DH 64, two at DH 128)
     // that take them largest first from the stream's work-queue counter.
-    const size_t bytes = sizeof(float) * (size_t)flash_slot_floats(dh) * (size_t)a.items * a.nheads;
+    // A captured call has a counter of its own behind them, cleared in the
+    // graph, and runs unsplit where there is no memory for the partials.
+    const size_t bytes =
+        Workspace::rounded(sizeof(float) * (size_t)flash_slot_floats(dh) * (size_t)a.items * a.nheads);
+    if (!wsf.room(bytes + 256)) {
+        a.chunk = full;
+        a.items = a.nqg;
+        return hip_status(launch_flash_attn(a, dh, s));
+    }
     char* ws = nullptr;
-    hipError_t e = wsf.get(&ws, bytes);
+    hipError_t e = wsf.get(&ws, bytes + 256);
     if (e != hipSuccess) return hip_status(e);
     a.part = reinterpret_cast<float*>(ws);
-    a.queue = flash_queue_of(s, e);
+    const bool graph = wsf.capturing();
+    if (graph) {
+        a.queue = reinterpret_cast<int*>(ws + bytes);
+        e = launch_flash_queue_reset(a.queue, s);
+    } else {
+        a.queue = flash_queue_of(s, e);
+    }
     if (e != hipSuccess) {
         (void)wsf.put(ws);
         return hip_status(e);
@@ -2008,7 +2087,7 @@ static int flash_launch(FlashArgs& a, int dh, Workspace& wsf) {
     e = launch_flash_attn(a, dh, s);
     // a launch that failed may leave the counter off zero: the next call
     // allocates and clears a new one
-    if (e != hipSuccess) (void)flash_queue_release(s);
+    if (e != hipSuccess && !graph) (void)flash_queue_release(s);
     const hipError_t f = wsf.put(ws);
     return hip_status(e != hipSuccess ? e : f);
 }

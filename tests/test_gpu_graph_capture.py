@@ -15,7 +15,11 @@ The cases use each kind of temporary the entry point carves from its region:
 split-K partial slabs (a TN product with beta = 1), the column partials of the
 GELU backward, the binary16 copy of an fp32 activation (AMP product wider
 than the in-kernel conversion serves), and none (bias + GELU on the 256 x 256
-tiles)."""
+tiles).
+
+The other two tests record the entry points that take their temporaries from
+the stream's workspace block: a graph must not hold memory that later calls on
+the stream use, outgrow or free, nor allocate any."""
 import ctypes
 
 import pytest
@@ -123,4 +127,110 @@ def test_noalloc_graph_replays(lib, case):
             f"{case}: replay {rep}: {int((C != want).sum())} outputs differ from the eager call"
         if want_cs:
             assert torch.equal(_bits(cs), _bits(want_sums)), f"{case}: replay {rep}: column sums differ"
+    del graph
+
+
+def _ordinary(case, g):
+    """The call and its output tensors."""
+    from logos_amd import vedic
+
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g, device="cuda") * std  # noqa: E731
+    if case == "splitk_f32":  # 128 tiles of 128 x 128 in slices of K
+        A, B, C = r(2048, 2048), r(2048, 1024, std=0.02), torch.empty(2048, 1024, device="cuda")
+        return lambda: vedic.gemm(vedic.OP_NN, A, B, C), [C]
+    if case == "splitk_f16_colsum":
+        A, B, C = r(8192, 512).half(), r(8192, 512, std=0.01).half(), torch.empty(512, 512, device="cuda")
+        cs = torch.empty(512, device="cuda")
+        return lambda: vedic.gemm(vedic.OP_TN, A, B, C, colsum=cs), [C, cs]
+    if case == "amp_cast":
+        A, B, C = r(2100, 4096), r(4096, 1024, std=0.02).half(), torch.empty(2100, 1024, device="cuda")
+        return lambda: vedic.amp_gemm(A, B, out=C), [C]
+    dh = int(case.split("_")[-1])
+    Q, K, V, dO = (r(1500, dh) for _ in range(4))
+    O, lse = torch.empty_like(Q), torch.empty(1500, device="cuda")
+    if case.startswith("attention_fwd"):  # one head: key chunks from the work queue, partials merged
+        return lambda: vedic.flash_attention_fwd(Q, K, V, O, lse=lse), [O, lse]
+    vedic.flash_attention_fwd(Q, K, V, O, lse=lse)
+    d = [torch.empty_like(Q) for _ in range(3)]
+    return lambda: vedic.flash_attention_bwd(Q, K, V, O, dO, lse, *d), d
+
+
+@pytest.mark.parametrize("case", ["splitk_f32", "splitk_f16_colsum", "amp_cast", "attention_fwd_64", "attention_fwd_128",
+                                  "attention_fwd_80", "attention_bwd_64"])
+def test_block_of_a_capture(lib, case):
+    """One eager call on the stream, then its capture, which takes the block
+    over; between the replays the stream serves other calls from a new one."""
+    from logos_amd import vedic
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(13)
+    call, outs = _ordinary(case, g)
+    oA, oB = torch.randn(4096, 640, generator=g, device="cuda"), torch.randn(4096, 512, generator=g, device="cuda")
+    oC = torch.empty(640, 512, device="cuda")
+    oQ, oK, oV = (torch.randn(2000, 64, generator=g, device="cuda") for _ in range(3))
+    oO = vedic.flash_attention_fwd(oQ, oK, oV)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        call()
+    torch.cuda.synchronize()
+    want = [t.clone() for t in outs]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        call()
+    for rep in range(4):
+        with torch.cuda.stream(stream):
+            vedic.gemm(vedic.OP_TN, oA, oB, oC)
+            got = vedic.flash_attention_fwd(oQ, oK, oV)
+        for t in outs:
+            t.fill_(7.0)
+        torch.cuda.synchronize()
+        assert torch.equal(got, oO)
+        graph.replay()
+        torch.cuda.synchronize()
+        for t, w in zip(outs, want):
+            assert torch.equal(_bits(t), _bits(w)), f"{case}: replay {rep}: {int((t != w).sum())} outputs differ"
+    del graph
+    assert lib.vedic_workspace_release(stream.cuda_stream) == _lib.STATUS_OK
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("case", ["splitk_f32", "splitk_f16_colsum", "amp_cast", "attention_fwd_64", "attention_fwd_80",
+                                  "attention_bwd_64"])
+def test_capture_without_a_block(lib, case):
+    """Captured on a stream that has no block: products and attention run
+    without slices, the AMP product converts in the kernel (the same bits), and
+    what cannot do without memory is refused, with nothing recorded."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(17)
+    call, outs = _ordinary(case, g)
+    call()
+    torch.cuda.synchronize()
+    want = [t.clone() for t in outs]
+    stream = torch.cuda.Stream()
+    lib.vedic_workspace_release(stream.cuda_stream)  # (the handle may have served another test)
+    torch.cuda.synchronize()
+    x = torch.zeros(4, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    refused = False
+    with torch.cuda.graph(graph, stream=stream):
+        x.add_(1.0)
+        try:
+            call()
+        except RuntimeError:
+            refused = True
+    assert refused == (case in ("splitk_f16_colsum", "attention_fwd_80", "attention_bwd_64"))
+    for t in outs:
+        t.fill_(7.0)
+    for rep in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float(x[0]) == rep + 1
+        for t, w in zip(outs, want):
+            if refused:
+                assert bool((t == 7.0).all())
+            elif case == "amp_cast":
+                assert torch.equal(_bits(t), _bits(w))
+            else:  # (the sums in another order)
+                assert float((t - w).abs().max()) <= 1e-5 * float(w.abs().max())
     del graph
