@@ -326,15 +326,14 @@ __device__ __forceinline__ void mfma_stage(const char* la, const char* lb, int a
     constexpr int KS = KN;
     constexpr int NR = (A_KC && !A32 ? MI : 2 * MI) + (B_KC ? NI : 2 * NI);  // LDS reads per k step
     constexpr int NM = MI * NI;                                              // MFMAs per k step
-    auto read_a = [&](int i, int kk) {
-        if constexpr (A32) return read_frag_a32<BK>(la, ar0 + 32 * i, kk, lane);
-        else return read_frag<A_KC, BM, BK>(la, ar0 + 32 * i, kk, lane);
-    };
     static_assert(NV <= KS * NM, "at most one load per MFMA");
     constexpr int EV = NV == 0 || NV * EVERY <= KS * NM ? EVERY : KS * NM / NV;  // spacing that fits
     half8_t af[2][MI], bf[2][NI];
 #pragma unroll
-    for (int i = 0; i < MI; ++i) af[0][i] = read_a(i, kk0);
+    for (int i = 0; i < MI; ++i) {
+        if constexpr (A32) af[0][i] = read_frag_a32<BK>(la, ar0 + 32 * i, kk0, lane);
+        else af[0][i] = read_frag<A_KC, BM, BK>(la, ar0 + 32 * i, kk0, lane);
+    }
 #pragma unroll
     for (int j = 0; j < NI; ++j) bf[0][j] = read_frag<B_KC, BN, BK>(lb, bc0 + 32 * j, kk0, lane);
 #pragma unroll
@@ -342,7 +341,10 @@ __device__ __forceinline__ void mfma_stage(const char* la, const char* lb, int a
         const int c = kk & 1, n = c ^ 1;
         if (kk + 1 < KS) {
 #pragma unroll
-            for (int i = 0; i < MI; ++i) af[n][i] = read_a(i, kk0 + kk + 1);
+            for (int i = 0; i < MI; ++i) {
+                if constexpr (A32) af[n][i] = read_frag_a32<BK>(la, ar0 + 32 * i, kk0 + kk + 1, lane);
+                else af[n][i] = read_frag<A_KC, BM, BK>(la, ar0 + 32 * i, kk0 + kk + 1, lane);
+            }
 #pragma unroll
             for (int j = 0; j < NI; ++j) bf[n][j] = read_frag<B_KC, BN, BK>(lb, bc0 + 32 * j, kk0 + kk + 1, lane);
         }
@@ -441,6 +443,25 @@ __device__ __forceinline__ const T* gathered_tile(const GemmArgs& a, int m0, int
         else                                                                             \
             sa.load(VEDIC_A_TILE(k_), (la), wave, lane, it.ke - k_);                     \
         sb.load(VEDIC_B_TILE(k_), (lb), wave, lane, it.ke - k_);                         \
+    } while (0)
+// Stage kt's MFMAs, and with HO the end of its head.  (A macro and, in
+// mfma_stage, no lambda around the fragment reads: captured by reference, the
+// addresses were no longer folded into the LDS reads' offsets -- TN 256 x 256
+// 30 -> 72 VALU instructions per stage, and spills in its generic epilogue.)
+#define VEDIC_MULTIPLY(kt, as, bs)                                                                                   \
+    do {                                                                                                             \
+        if constexpr (HO == 1) {                                                                                     \
+            mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, true, A32D>(as, bs, wm * WM, wn * WN, lane, acc);      \
+            head_done();                                                                                             \
+        } else {                                                                                                     \
+            mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, false, A32D>(as, bs, wm * WM, wn * WN, lane, acc,      \
+                                                                             wk * KN);                                \
+            if (HO == 2 && ((kt) + 1) % seg == 0) {                                                                  \
+                head_done();                                                                                         \
+                _Pragma("unroll") for (int i = 0; i < MI; ++i)                                                       \
+                    _Pragma("unroll") for (int j = 0; j < NI; ++j) acc[i][j] = float16_t{};                          \
+            }                                                                                                        \
+        }                                                                                                            \
     } while (0)
 // The first ST - 1 stages of a work item; with an fp32 A in registers each
 // stage's A is committed as soon as it has landed (its B may still be in flight).
@@ -562,24 +583,6 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
             bias_pre[j] = pre_bias && col < args.N ? args.bias[col] : 0.0f;
         }
 
-        // Stage kt's MFMAs, and with HO the end of its head.
-        auto multiply = [&](const char* as, const char* bs, int kt) {
-            if constexpr (HO == 1) {
-                mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, true, A32D>(as, bs, wm * WM, wn * WN, lane, acc);
-                head_done();
-            } else {
-                mfma_stage<A_KC, B_KC, BM, BN, BK, MI, NI, 0, 1, KN, false, A32D>(as, bs, wm * WM, wn * WN, lane, acc,
-                                                                                 wk * KN);
-                if (HO == 2 && (kt + 1) % seg == 0) {
-                    head_done();
-#pragma unroll
-                    for (int i = 0; i < MI; ++i)
-#pragma unroll
-                        for (int j = 0; j < NI; ++j) acc[i][j] = float16_t{};
-                }
-            }
-        };
-
         // Uniform pipeline: every stage step waits for the same number of
         // loads and issues stage kt + ST - 1, which past the work item's
         // range loads zeros without touching memory; only the MFMAs are
@@ -607,7 +610,7 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
                     // register loads, then the MFMAs, then the conversion into
                     // stage kt - 1's buffer, free since the barrier above
                     VEDIC_ISSUE(kt + ST - 1, As[sl], Bs[sl]);
-                    if (kt < nk) multiply(As[s], Bs[s], kt);
+                    if (kt < nk) VEDIC_MULTIPLY(kt, As[s], Bs[s]);
                     wait_vmcnt<SB::NLD>();
                     sa.commit(As[sl], wave, lane);
                 } else if constexpr (kInterleave) {
@@ -620,7 +623,13 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
                     }
                 } else {
                     VEDIC_ISSUE(kt + ST - 1, As[sl], Bs[sl]);
-                    if (kt < nk) multiply(As[s], Bs[s], kt);
+                    if constexpr (A32D && HO == 0) {
+                        // (here a lambda is the faster: 1500 x 1024 x 1024 18.8 us, 19.2 without)
+                        auto multiply = [&](const char* as, const char* bs) { VEDIC_MULTIPLY(kt, as, bs); };
+                        if (kt < nk) multiply(As[s], Bs[s]);
+                    } else {
+                        if (kt < nk) VEDIC_MULTIPLY(kt, As[s], Bs[s]);
+                    }
                 }
             }
         }
@@ -720,6 +729,7 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
     wait_vmcnt<0>();  // the trailing zero loads still write LDS
 }
 
+#undef VEDIC_MULTIPLY
 #undef VEDIC_ISSUE
 #undef VEDIC_PROLOGUE
 #undef VEDIC_PROLOGUE_STAGE

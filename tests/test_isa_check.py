@@ -3,6 +3,7 @@ no 12- or 16-byte store has a data register rewritten by a VALU instruction
 within four wait states (twice the gfx940-family rule), and the scanner
 itself finds such a rewrite when one is planted in a disassembly."""
 import os
+import re
 
 import pytest
 
@@ -17,6 +18,26 @@ def test_library_wide_stores_keep_the_margin():
     total, found = isa_check.scan(LIB)
     assert total > 0  # the flash, layernorm and reduction kernels store 16 bytes
     assert found == [], found[:5]
+
+
+def test_fp16_gemm_kernels_do_not_spill():
+    """No scratch access in any binary16 GEMM kernel (the generic epilogue of the
+    NN 256 x 256 tile has one register pair's store and load): addresses that
+    are no longer folded into the LDS reads show up as spills there first."""
+    if not os.path.exists(LIB):
+        pytest.skip("library not built")
+    count, kernels = {}, set()
+    for text in isa_check.disassemble(LIB):
+        name = None
+        for line in text.splitlines():
+            m = re.match(r"^[0-9a-f]+ <(.+)>:$", line)
+            if m:
+                name = m.group(1)
+                kernels.add(name)
+            elif "scratch_" in line and re.match(r"\s*scratch_(load|store)", line):
+                count[name] = count.get(name, 0) + 1
+    assert sum("gemm_f16_kernel" in k for k in kernels) > 100
+    assert {k: n for k, n in count.items() if "gemm_f16_kernel" in k and n > 2} == {}
 
 
 _PLANT = """
