@@ -497,7 +497,8 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
     constexpr int WMN = WGM * WGN, NW = WMN * WGK, WM = BM / WGM, WN = BN / WGN, MI = WM / 32, NI = WN / 32;
     constexpr int KN = BK / 16 / WGK;
     static_assert(KN * WGK * 16 == BK, "the k steps of a stage divide among the wave groups");
-    constexpr bool A32 = OP == 3, A32D = A32 && BM == 128, A32R = A32 && !A32D;  // an fp32 A: in LDS, in registers
+    // (op 4 is op 3 with A in registers on 128 x 128 tiles too: gathered A, few tiles)
+    constexpr bool A32 = OP >= 3, A32D = OP == 3 && BM == 128, A32R = A32 && !A32D;  // an fp32 A: in LDS, in registers
     constexpr bool A_KC = OP != 2, B_KC = OP == 1;
     using SA = std::conditional_t<A32R, SideA32<BM, BK, NW>,
                                   std::conditional_t<A32D, SideA32D<BM, BK, NW>, Side<A_KC, BM, BK, NW>>>;
@@ -509,7 +510,7 @@ __global__ void __launch_bounds__(WGM* WGN * WGK * 64) gemm_f16_kernel(GemmArgs 
     // of issued together (2-3 % faster: fewer waves held at a full
     // texture-address queue); 128 x 128 tiles measured slower that way.
     constexpr bool kInterleave = BM * BN >= 256 * 256 && WGK == 1 && HO == 0 && !A32;
-    static_assert(HO == 0 || (WGK == 1 && (OP == 0 || OP == 3)), "gathered A: NN or AMP, one k group");
+    static_assert(HO == 0 || (WGK == 1 && (OP == 0 || OP >= 3)), "gathered A: NN or AMP, one k group");
 
     // One LDS object per stage (A then B): reads of one stage provably do not
     // alias the direct loads into another.  The compiler follows only a few

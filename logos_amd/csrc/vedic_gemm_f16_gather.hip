@@ -25,6 +25,8 @@ VEDIC_F16_KERNEL_HO(3, CfgMid, 1);
 VEDIC_F16_KERNEL_HO(3, CfgMid, 2);
 VEDIC_F16_KERNEL_HO(3, CfgSmall, 1);
 VEDIC_F16_KERNEL_HO(3, CfgSmall, 2);
+VEDIC_F16_KERNEL_HO(4, CfgSmall, 1);
+VEDIC_F16_KERNEL_HO(4, CfgSmall, 2);
 
 namespace {
 
@@ -39,6 +41,16 @@ template <int OP>
 hipError_t launch_gather_op(const GemmArgs& a, hipStream_t s) {
     const int cus = device_cu_count();
     if (f16_tile_estimate(a.M, a.N, cus, 1) <= f16_tile_estimate(a.M, a.N, cus, 2)) return launch_ho<OP, CfgMid>(a, s);
+    // An fp32 A on a few tiles goes through registers (op 4), not through LDS:
+    // with a workgroup on less than a quarter of the CUs the stages are not
+    // bound by the rate of the loads but by their own steps, and converting a
+    // value once per workgroup is the shorter step (16 heads of 64 x 1024: 512
+    // rows, 32 tiles, 22.8 against 23.6 us; 700 rows, 48 tiles, 23.1 / 24.0; 1000
+    // rows, 64 tiles, 25.7 / 24.0; 8 heads of 128: 24.7 / 25.9, 25.2 / 26.4, 26.5 / 26.5).
+    if constexpr (OP == 3) {
+        const int64_t tiles = (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128);
+        if (tiles * 4 < cus) return launch_ho<4, CfgSmall>(a, s);
+    }
     return launch_ho<OP, CfgSmall>(a, s);
 }
 

@@ -84,6 +84,10 @@ def test_gather_full_size(amp):
 @pytest.mark.parametrize("M,N,hc,nheads,amp", [
     (8192, 1024, 128, 8, True),     # DH 128: two stages per head
     (1000, 1024, 64, 16, False),    # rows not a multiple of the tile
+    (100, 1024, 64, 16, True),      # fp32 heads on 8, 56 and 64 tiles of 128 x 128: in registers below a quarter of the CUs
+    (769, 1000, 128, 8, True),
+    (897, 1024, 64, 16, True),
+    (33, 72, 64, 3, True),
     (300, 200, 64, 3, True),        # columns not a multiple of the tile
     (256, 256, 64, 4, False),       # small: 128 x 128 tiles
     (512, 1536, 64, 4, True),       # fp32 heads with N > 1024: cast into the workspace first
