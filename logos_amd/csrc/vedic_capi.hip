@@ -495,15 +495,15 @@ static hipError_t launch_f32_tiled(int op, bool vec, const GemmArgs& a, hipStrea
 // 1 = no split.
 //
 // fp32 products on the split kernel (f32_use_split) with 128 x 128 tiles for
-// half the CUs or more, but not for all: slices of at least 384 steps up to
+// half the CUs or more, but not for all (f32s_mid_tiles): slices of at least 384 steps up to
 // the three workgroups a CU holds (2048 x 1024 x 1024 NN, 128 tiles: 47.8 us
 // unsplit, 35.3 in two slices, 37.2 in four; 1001 x 1999 x 2047 TN 89.0, 60.6,
 // 60.4), within kSplitBytes of partials, so that a caller with a fixed scratch
 // region is never refused for them.
 static constexpr int64_t kSplitBytes = int64_t(24) << 20;
-static int choose_ksplit(int M, int N, int K, int cus, bool f16) {
+static int choose_ksplit(int op, int M, int N, int K, bool vec, int cus, bool f16) {
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-    if (!f16 && t128 * 2 >= cus && f32_use_split(M, N, K, true, cus)) {
+    if (!f16 && t128 * 2 >= cus && f32s_mid_tiles(M, N, K, cus) && f32_use_split(op, M, N, K, vec, false, cus)) {
         if (t128 >= cus) return 1;
         int64_t s = 3 * (int64_t)cus / t128;
         s = s < K / 384 ? s : K / 384;
@@ -779,7 +779,7 @@ static int gemm_impl(const vedic_gemm_desc_t* d, float* const* heads, int nheads
     const bool wave_split = !f16 && direct && d->op != VEDIC_OP_TN && f32_wave_split(d->M, d->N, device_cu_count());
     int ks = skinny || scatter || wave_split || (f16 && !direct)
                  ? 1
-                 : choose_ksplit(d->M, d->N, d->K, device_cu_count(), f16);
+                 : choose_ksplit(d->op, d->M, d->N, d->K, vec, device_cu_count(), f16);
     // (in a capture without memory for the slices the product runs unsplit)
     if (ks > 1 && !ws.room(sizeof(float) * (size_t)d->M * d->N * ks +
                            (d->colsum ? Workspace::rounded(sizeof(float) * colsum_matrix_floats(d->M, d->N)) : 0)))
@@ -1682,7 +1682,7 @@ extern "C" int vedic_gemm_gather(const vedic_gemm_desc_t* d, const void* const* 
     // output over its head's k range, as the head-ordered kernels do: not on
     // the narrow tiles (N <= 64) or the decode kernel (M <= 32), whose waves
     // split the contraction and add partials, nor split over K.
-    const bool chain = d->N > 64 && d->M > 32 && choose_ksplit(d->M, d->N, head_cols, device_cu_count(), true) == 1;
+    const bool chain = d->N > 64 && d->M > 32 && choose_ksplit(d->op, d->M, d->N, head_cols, true, device_cu_count(), true) == 1;
     if (!heads_ok || !b_ok || !chain) {
         // the per-head products themselves
         const int64_t n = (int64_t)d->M * d->N;

@@ -117,23 +117,37 @@ inline bool f32_wave_split(int M, int N, int cus) {
     return t64 < cus && t32 * 2 >= cus;
 }
 
-// Whether an fp32 product runs on the bf16 split kernel (vedic_gemm_f32s.hpp)
-// rather than on v_mfma_f32_32x32x2_f32 (vedic_gemm_f32.hpp).  The split
-// kernel's stage of 16 steps costs a CU about 0.7 us alone whatever the tile,
-// so it wants tiles for half the CUs and, where it has no more, a contraction
-// long enough to be split over workgroups: 2048 x 1024 (128 tiles of 128 x 128)
-// K = 1024 35.3 / 35.7 / 35.0 us (NN / NT / TN) against 38.4 / 35.8 / 43.3, but
-// K = 256 15.2 / 14.0 / 15.6 against 12.5 / 12.0 / 13.6; 1024 x 1024 x 1024 (64
-// tiles, four slices) 25.9 / 25.3 / 26.2 against 25.6 / 21.2 / 29.0; from 192
-// tiles up it is faster throughout (4096 x 1024 x 256 16.7 against 23.0).
-// Rows that are not 16-byte aligned, which the other kernel cannot load, always
-// run on it (512 x 1000 x 1000 with a pitch of 1001: 29.7 against 70.9 us on
-// the element-wise kernel).
-inline bool f32_use_split(int M, int N, int K, bool vec, int cus) {
-    if (!vec) return true;
+// Whether the bf16 split kernel (vedic_gemm_f32s.hpp) runs an fp32 product on
+// tiles of 128 x 128 or more: outputs of that many tiles for more than half the
+// CUs, or for half of them with a contraction of 512 or more.  Its stage of 16
+// steps costs a CU about 0.7 us alone whatever the tile.
+inline bool f32s_mid_tiles(int M, int N, int K, int cus) {
     if (N <= 64) return false;
     const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     return tiles * 2 > cus || (tiles * 2 == cus && K >= 512);
+}
+
+// Whether an fp32 product runs on that kernel rather than on
+// v_mfma_f32_32x32x2_f32 (vedic_gemm_f32.hpp).  With tiles for more than half the
+// CUs it is faster throughout (1100 x 1920 x 64, 135 tiles, 7.5 us against 10.0;
+// 2176 x 1024 x 512 25.7 / 39.4; 4096 x 1024 x 256 16.7 / 23.0).  With tiles for half
+// of them the contraction has to be split over workgroups (choose_ksplit) and
+// long: 2048 x 1024 (128 tiles) NN / NT / TN, this kernel against the other,
+// K = 512 25.2 / 23.3 / 26.0 us against 21.6 / 20.6 / 23.8; 640 30.5 / 27.9 / 31.1
+// against 25.5 / 24.1 / 28.6; 768 (two slices from here on) 33.5 / 32.1 / 31.9
+// against 29.8 / 28.0 / 33.5; 900 34.4 / 33.8 / 33.5 against 36.1 / 33.6 / 40.0; 1024
+// 34.9 / 35.1 / 34.2 against 38.5 / 35.9 / 43.4.  Scattered outputs are not split
+// (NN K = 1024 48.5 against 38.9).  Fewer tiles: 1024 x 1024 x 1024 (64, four
+// slices) 25.9 / 25.3 / 26.2 against 25.6 / 21.2 / 29.0.
+// Rows that are not 16-byte aligned, which the other kernel cannot load, always
+// run here (512 x 1000 x 1000 with a pitch of 1001: 29.7 against 70.9 us on the
+// element-wise kernel).
+inline bool f32_use_split(int op, int M, int N, int K, bool vec, bool scatter, int cus) {
+    if (!vec) return true;
+    if (!f32s_mid_tiles(M, N, K, cus)) return false;
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    if (tiles * 2 != cus) return true;
+    return !scatter && K >= (op == 0 ? 896 : op == 1 ? 1024 : 768);
 }
 
 struct GemmArgs {

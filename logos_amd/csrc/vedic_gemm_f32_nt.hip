@@ -13,7 +13,7 @@ VEDIC_F32S_KERNEL(1, false, CfgSMid, EK_GENERIC);
 VEDIC_F32S_KERNEL(1, false, CfgSSmall, EK_GENERIC);
 
 hipError_t launch_gemm_f32_direct_nt(bool vec, const GemmArgs& a, hipStream_t s) {
-    if (!f32_use_split(a.M, a.N, a.K, vec, device_cu_count())) return launch_gemm_f32_mfma_op<1>(a, s);
+    if (!f32_use_split(1, a.M, a.N, a.K, vec, a.head_cols > 0, device_cu_count())) return launch_gemm_f32_mfma_op<1>(a, s);
     return vec ? launch_gemm_f32s_op<1, true>(a, s) : launch_gemm_f32s_op<1, false>(a, s);
 }
 

@@ -11,7 +11,7 @@ VEDIC_F32S_KINDS(2, CfgSMid);
 VEDIC_F32S_KINDS(2, CfgSSmall);
 
 hipError_t launch_gemm_f32_direct_tn(bool vec, const GemmArgs& a, hipStream_t s) {
-    if (!f32_use_split(a.M, a.N, a.K, vec, device_cu_count())) return launch_gemm_f32_mfma_op<2>(a, s);
+    if (!f32_use_split(2, a.M, a.N, a.K, vec, a.head_cols > 0, device_cu_count())) return launch_gemm_f32_mfma_op<2>(a, s);
     return launch_gemm_f32s_op<2, true>(a, s);
 }
 

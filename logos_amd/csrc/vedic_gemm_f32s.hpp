@@ -395,7 +395,7 @@ hipError_t launch_gemm_f32s_op(const GemmArgs& a, hipStream_t s) {
         if constexpr (OP != 2) return launch_f32s_kind<OP, VEC, CfgSMid>(a, s);
     }
     // (TN, whose kernels take any alignment, and unaligned rows: few tiles too)
-    if (!f32_use_split(a.M, a.N, a.K, true, cus)) return launch_f32s_kind<OP, VEC, CfgSSmall>(a, s);
+    if (!f32s_mid_tiles(a.M, a.N, a.K, cus)) return launch_f32s_kind<OP, VEC, CfgSSmall>(a, s);
     return launch_f32s_kind<OP, VEC, CfgSMid>(a, s);
 }
 

@@ -21,8 +21,8 @@ def _operands(rng, layout, M, N, K):
     return A, B
 
 
-# (M, N, K): 128 x 128 tiles (129 tiles and up, or 128 of them with K >= 512,
-# then split over K), 256 x 256 tiles, ragged edges, one step to several stage
+# (M, N, K): 128 x 128 tiles (129 tiles and up, or 128 of them with a K that is
+# split over workgroups, here 1160), 256 x 256 tiles, ragged edges, one step to several stage
 # groups of the contraction
 SHAPES = [(2049, 1025, 1), (2177, 1100, 16), (2100, 1160, 17), (1999, 2055, 33), (2048, 1024, 512), (1930, 1024, 1160),
           (3588, 3700, 40), (3841, 3585, 33)]
