@@ -136,41 +136,78 @@ __device__ __forceinline__ SplitFrag read_split(const char* lds, int rc0, int la
 
 // A wave's (32 MI) x (32 NI) block on v_mfma_f32_32x32x2_f32 from unscaled
 // global values: for blocks whose split sums are not finite (an operand of
-// 2^104 or more, an infinity, a NaN, a result past 2^80).  Element loads, no
-// LDS, no barrier.
+// 2^104 or more, an infinity, a NaN, a result past 2^80).  No LDS, no barrier: 2 Q steps' values of all the block's rows and
+// columns are in flight together (lane half h takes steps Q h .. Q h + Q - 1 of
+// them; Q = 4 where the accumulators leave no more registers), and feed Q MI NI
+// MFMAs.  8192 x 8192 x 1024 all NaN NN / NT / TN 5732 /
+// 7513 / 3797 -> 1853 / 1618 / 1996 us, of which the split pass is 605 (1003 / 963 /
+// 1066 on gemm_f32_kernel); one NaN 2817 / 2585 / 2339 -> 1063 / 916 / 1152.
 template <bool A_KC, bool B_KC, int MI, int NI>
 __device__ __forceinline__ void f32_block_slow(const GemmArgs& args, int row0, int col0, int kb, int ke, int lane,
                                                float16_t (&acc)[MI][NI]) {
+    constexpr int Q = MI * NI > 4 ? 4 : 8;
     const int l32 = lane & 31, h = lane >> 5;
     const float* A = static_cast<const float*>(args.A);
     const float* B = static_cast<const float*>(args.B);
+    const int64_t ka = A_KC ? 1 : args.lda, kn = B_KC ? 1 : args.ldb;
+    const float* pa[MI];
+    const float* pb[NI];
+    // (rows and columns past M and N repeat the last: not stored)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int r = min(row0 + 32 * i + l32, args.M - 1);
+        pa[i] = (A_KC ? A + (int64_t)r * args.lda : A + r) + (kb + Q * h) * ka;
+    }
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+        const int n = min(col0 + 32 * j + l32, args.N - 1);
+        pb[j] = (B_KC ? B + (int64_t)n * args.ldb : B + n) + (kb + Q * h) * kn;
+    }
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-            // (rows and columns past M and N repeat the last: not stored)
-            const int r = min(row0 + 32 * i + l32, args.M - 1), n = min(col0 + 32 * j + l32, args.N - 1);
-            const float* pa = A_KC ? A + (int64_t)r * args.lda : A + r;
-            const float* pb = B_KC ? B + (int64_t)n * args.ldb : B + n;
-            const int64_t ka = A_KC ? 1 : args.lda, kb_ = B_KC ? 1 : args.ldb;
-            float16_t t = float16_t{};
+        for (int j = 0; j < NI; ++j) acc[i][j] = float16_t{};
+    int k = kb;
 #pragma unroll 1
-            for (int k = kb; k < ke; k += 16) {  // 16 steps' loads in flight
-                float x[8], y[8];
+    for (; k + 2 * Q <= ke; k += 2 * Q) {
+        float x[MI][Q], y[NI][Q];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int kk = min(k + 2 * q + h, ke - 1);
-                    x[q] = pa[kk * ka];
-                    y[q] = pb[kk * kb_];
-                }
+        for (int i = 0; i < MI; ++i) {
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const bool in = k + 2 * q + h < ke;
-                    t = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x[q] : 0.0f, in ? y[q] : 0.0f, t, 0, 0, 0);
-                }
-            }
-            acc[i][j] = t;
+            for (int q = 0; q < Q; ++q) x[i][q] = pa[i][q * ka];
+            pa[i] += 2 * Q * ka;
         }
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) y[j][q] = pb[j][q * kn];
+            pb[j] += 2 * Q * kn;
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][q], y[j][q], acc[i][j], 0, 0, 0);
+    }
+    // the last steps, fewer than 2 Q: those past the end load the last one and count as zeros
+#pragma unroll 1
+    for (int q = 0; q < Q && k + q < ke; ++q) {
+        const bool in = k + Q * h + q < ke;
+        const int64_t d = in ? q : ke - 1 - (k + Q * h);
+        float x[MI], y[NI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) x[i] = pa[i][d * ka];
+#pragma unroll
+        for (int j = 0; j < NI; ++j) y[j] = pb[j][d * kn];
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+                acc[i][j] =
+                    __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x[i] : 0.0f, in ? y[j] : 0.0f, acc[i][j], 0, 0, 0);
+    }
 }
 
 template <int OP, bool VEC, int BM, int BN, int WGM, int WGN, int WPE, int SETS, int KIND>

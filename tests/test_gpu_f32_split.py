@@ -142,3 +142,49 @@ def test_nonfinite(opname):
     assert np.array_equal(got[inf], want[inf])
     fin = np.isfinite(want)
     assert np.all(np.abs(got[fin] - want[fin]) <= 4 * np.sqrt(K) * o.U32 * K * 30)
+
+
+# (M, N, K, element offset of the operands): 256 x 256 tiles; 128 x 128 tiles in
+# slices of K, unsplit with a ragged last group, unaligned; 64 x 64 tiles in slices, unaligned
+REPEAT = [(3841, 3585, 81, 0), (1930, 1024, 1160, 0), (2177, 1100, 300, 0), (2100, 1160, 47, 1), (130, 700, 2000, 1)]
+
+
+@pytest.mark.parametrize("opname", list(OPS))
+@pytest.mark.parametrize("shape", REPEAT, ids=lambda s: "x".join(map(str, s)))
+def test_repeat(opname, shape):
+    """Blocks repeated on the fp32 MFMA in every tile configuration, beside
+    blocks that are not: an infinity and a NaN at steps past the middle (with
+    slices only a later one repeats), a row of 2^110 and a column of 2^60
+    against a row of 2^40 (a result past 2^80)."""
+    from logos_amd import vedic
+
+    layout = OPS[opname]
+    M, N, K, off = shape
+    rng = np.random.default_rng(zlib.crc32(f"f32s-repeat-{opname}-{shape}".encode()))
+    A, B = normal(rng, (M, K)), normal(rng, (K, N))
+    A[5, K - 2], A[M - 1, K // 2 + 1] = np.inf, np.nan
+    A[M // 2] *= np.float32(2.0 ** 110)
+    A[M // 2 + 1] *= np.float32(2.0 ** 40)
+    B[:, N // 3] *= np.float32(2.0 ** 60)
+    A[M // 2, :] *= np.float32(2.0 ** -55)
+    A[M // 2, 0] = np.float32(2.0 ** 110)
+
+    def put(X):
+        t = torch.zeros((X.shape[0], X.shape[1] + 2 * off), device="cuda")
+        t[:, off:off + X.shape[1]] = dev(np.ascontiguousarray(X))
+        return t[:, off:off + X.shape[1]]
+
+    C0 = normal(rng, (M, N))
+    a, b = put(A.T if layout == o.TN else A), put(B.T if layout == o.NT else B)
+    got = host(vedic.gemm(layout, a, b, dev(C0), beta=1.0)).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        A64, B64 = A.astype(np.float64), B.astype(np.float64)
+        want = A64 @ B64 + C0
+        size = np.abs(A64) @ np.abs(B64) + np.abs(C0)
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    inf = np.isinf(want)
+    assert inf.any() and np.array_equal(got[inf], want[inf])
+    fin = ~nan & ~inf & (size < 3e38)
+    assert fin.sum() > 0.99 * (fin.size - nan.sum() - inf.sum())
+    assert np.all(np.abs(got[fin] - want[fin]) <= 4 * np.sqrt(K) * o.U32 * size[fin])
