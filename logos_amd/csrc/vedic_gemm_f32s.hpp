@@ -38,6 +38,11 @@ namespace vedic {
 
 constexpr int kSplitK = 16;         // contraction steps per stage
 constexpr int kSplitRowBytes = 96;  // 3 parts x 16 steps x 2 bytes
+// Sums of one or two products are repeated on the fp32 MFMA: the terms that the
+// split drops cost more there than its longer accumulation gains (largest error
+// of K = 1, 2, 3 in units of 2^-24 of the summed magnitudes 2.5, 2.8, 2.4 against
+// 1.0, 1.95, 2.5).
+constexpr int kSplitMinK = 3;
 
 __device__ __forceinline__ int split_half(int row, int h) { return (h ^ ((row >> 3) & 1)) << 4; }
 
@@ -136,7 +141,8 @@ __device__ __forceinline__ SplitFrag read_split(const char* lds, int rc0, int la
 
 // A wave's (32 MI) x (32 NI) block on v_mfma_f32_32x32x2_f32 from unscaled
 // global values: for blocks whose split sums are not finite (an operand of
-// 2^104 or more, an infinity, a NaN, a result past 2^80).  No LDS, no barrier: 2 Q steps' values of all the block's rows and
+// 2^104 or more, an infinity, a NaN, a result past 2^80) and for one or two
+// steps.  No LDS, no barrier: 2 Q steps' values of all the block's rows and
 // columns are in flight together (lane half h takes steps Q h .. Q h + Q - 1 of
 // them; Q = 4 where the accumulators leave no more registers), and feed Q MI NI
 // MFMAs.  8192 x 8192 x 1024 all NaN NN / NT / TN 5732 /
@@ -247,8 +253,10 @@ gemm_f32s_kernel(GemmArgs args) {
     SB sb;
     sa.init(tid, args.lda, it.m0, args.M);
     sb.init(tid, args.ldb, it.n0, args.N);
-    const int len = it.ke - it.kb, nk = (len + P * kSplitK - 1) / (P * kSplitK) * P;
-    const int rem = len - (nk - P) * kSplitK;
+    // (len 0, no stage at all, for the steps that f32_block_slow does alone)
+    const bool few = it.ke - it.kb < kSplitMinK;
+    const int len = few ? 0 : it.ke - it.kb, nk = (len + P * kSplitK - 1) / (P * kSplitK) * P;
+    const int rem = few ? 0 : len - (nk - P) * kSplitK;
     typename SA::Values va[SETS];
     typename SB::Values vb[SETS];
     auto load_first = [&](int kt) {  // kt < P
@@ -334,7 +342,7 @@ gemm_f32s_kernel(GemmArgs args) {
             acc[i][j] *= kSplitUnscale2;
             probe = nonfinite_probe(acc[i][j], probe);
         }
-    if (__any(probe != 0.0f))
+    if (few || __any(probe != 0.0f))
         f32_block_slow<A_KC, B_KC, MI, NI>(args, row0, col0, it.kb, it.ke, lane, acc);
     // split-K: this slice's raw partial goes to its own slab of the workspace
     void* const cp = args.ksplit > 1 ? static_cast<void*>(static_cast<float*>(args.C) + it.s * args.c_split_stride)

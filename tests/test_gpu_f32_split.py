@@ -51,6 +51,27 @@ def test_tiles(opname, shape, pad):
 
 
 @pytest.mark.parametrize("opname", list(OPS))
+@pytest.mark.parametrize("shape", [(2049, 1032), (2100, 1161), (200, 330), (8, 4)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("K", [1, 2, 3, 4])
+def test_few_steps(opname, shape, K):
+    """One product is rounded once, two products at most three times: no part
+    of a value may be dropped there.  From three on the split's bound is within
+    binary32 summation's (K roundings, and 2^-24 of each product dropped)."""
+    from logos_amd import vedic
+
+    layout = OPS[opname]
+    M, N = shape
+    rng = np.random.default_rng(zlib.crc32(f"f32s-few-{opname}-{shape}-{K}".encode()))
+    A, B = _operands(rng, layout, M, N, K)
+    got = host(vedic.gemm(layout, dev(A), dev(B)))
+    a, b = (A.T if layout == o.TN else A).astype(np.float64), (B.T if layout == o.NT else B).astype(np.float64)
+    if K == 1:
+        assert np.array_equal(got, (a @ b).astype(np.float32))
+    bound = {1: 1, 2: 2, 3: 4, 4: 5}[K] * o.U32 * (np.abs(a) @ np.abs(b))
+    assert np.all(np.abs(got - a @ b) <= bound)
+
+
+@pytest.mark.parametrize("opname", list(OPS))
 @pytest.mark.parametrize("shape", [(63, 65, 100), (200, 33, 300), (130, 700, 2000), (1, 64, 5), (40, 1, 1)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_small_unaligned(opname, shape):
