@@ -424,7 +424,12 @@ static hipError_t launch_f32s_kind(const GemmArgs& a, hipStream_t s) {
 // 256 x 256 tiles where their whole rounds cost less than the 128 x 128 tiles'
 // share per CU: a 256 x 256 round does four 128 x 128 tiles' work at 1.1 times
 // their rate (8192 x 8192 above; 8192 x 3072, 1.5 rounds, 254 against 246 us).
-inline bool f32s_large(int M, int N, int cus) {
+// Not for contractions of at most 64, which the writing of C bounds: three
+// workgroups on a CU overlap their epilogues, one does not (8192 x 4096 NT
+// accumulated, K = 4 59.0 us against 42.0, 64 65.9 / 47.4; 8192 x 8192 K = 4 59.9 /
+// 44.1, 64 75.4 / 72.0, 128 108.5 / 108.3, 256 176.4 / 186.3).
+inline bool f32s_large(int M, int N, int K, int cus) {
+    if (K <= 64) return false;
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     return (t256 + cus - 1) / cus * 4 * 10 < (t128 + cus - 1) / cus * 11;
@@ -435,7 +440,7 @@ hipError_t launch_gemm_f32s_op(const GemmArgs& a, hipStream_t s) {
     const int cus = device_cu_count();
     if constexpr (VEC) {
         // (256 rows of a longer leading dimension pass 32-bit offsets)
-        if (a.ksplit <= 1 && a.lda < kMaxLd / 2 && a.ldb < kMaxLd / 2 && f32s_large(a.M, a.N, cus))
+        if (a.ksplit <= 1 && a.lda < kMaxLd / 2 && a.ldb < kMaxLd / 2 && f32s_large(a.M, a.N, a.K, cus))
             return launch_f32s_kind<OP, VEC, CfgSLarge>(a, s);
         if constexpr (OP != 2) return launch_f32s_kind<OP, VEC, CfgSMid>(a, s);
     }

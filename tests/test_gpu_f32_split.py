@@ -25,7 +25,7 @@ def _operands(rng, layout, M, N, K):
 # split over workgroups, here 1160), 256 x 256 tiles, ragged edges, one step to several stage
 # groups of the contraction
 SHAPES = [(2049, 1025, 1), (2177, 1100, 16), (2100, 1160, 17), (1999, 2055, 33), (2048, 1024, 512), (1930, 1024, 1160),
-          (3588, 3700, 40), (3841, 3585, 33)]
+          (3588, 3700, 40), (3841, 3585, 33), (3588, 3700, 72), (3841, 3585, 65)]
 
 
 @pytest.mark.parametrize("opname", list(OPS))
@@ -91,7 +91,7 @@ def test_small_unaligned(opname, shape):
           alpha=0.5, beta=-2.0, C0=C0, label=f"{opname} {shape} alpha/beta")
 
 
-@pytest.mark.parametrize("shape", [(2100, 1160, 50), (3841, 3585, 33)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("shape", [(2100, 1160, 50), (3841, 3585, 33), (3841, 3585, 81)], ids=lambda s: "x".join(map(str, s)))
 def test_epilogues(shape):
     """Each fused epilogue on the 128 x 128 and 256 x 256 tiles."""
     from logos_amd import vedic
