@@ -565,10 +565,13 @@ constexpr int kOpAmp = 3;
 #endif
 constexpr int kAmpInKernelMaxN = VEDIC_AMP_IN_KERNEL_MAX_N;
 // Long contractions of more than 512 columns take the cast too: every tile
-// column reads the fp32 A again, and its 4 bytes per value bound the stages
-// (1531 x 1024 x 4096 41.3 us in the kernel, 6.7 + 25.5 cast + binary16 GEMM;
-// 8192 x 1024 x 4096 98.8, 27.8 + 67.6; but 512 x 1024 x 1024 17.9, 6.6 + 11.8,
-// and 4096 x 512 x 2048 27.5, 8.3 + 21.2).
+// column reads the fp32 A again, and its 4 bytes per value bound the stages.
+// In the kernel against the cast and the binary16 GEMM, us, at M = 33, 300, 1024,
+// 2100, 8192: N = 1024, K = 2048 20.6 / 16.6, 21.4 / 18.1, 22.7 / 21.7, 31.8 / 26.6,
+// 54.4 / 54.0; K = 4096 21.4 / 17.1, 22.4 / 19.5, 25.1 / 25.2, 57.5 / 43.0, 100.1 / 98.7;
+// K = 8192 22.5 / 18.4, 24.8 / 22.0, 39.6 / 36.8, 109.8 / 77.1, 257.6 / 205.2; N = 520,
+// K = 2048 20.8 / 16.6, 22.5 / 18.9, 22.9 / 21.4, 24.2 / 22.7, 51.5 / 45.9.  But 512 x 1024
+// x 1024 17.7 against 6.6 + 11.8, and 4096 x 512 x 2048 27.5 against 8.3 + 21.2.
 // (M <= 32 after the cast would run on the decode kernel, whose sums have
 // another order than the in-kernel conversion's.)
 static bool amp_cast_first(int M, int N, int K) {
@@ -768,7 +771,7 @@ static int gemm_impl(const vedic_gemm_desc_t* d, float* const* heads, int nheads
     Workspace& ws = wsp ? *wsp : pool;
     // (a caller's fixed scratch region is asked for a copy of A only where it
     // must, and a captured call does without where it can: the bits are the same)
-    if (amp && (!direct || (wsp ? d->N > kAmpInKernelMaxN : amp_cast_first(d->M, d->N, d->K))) &&
+    if (amp && (!direct || (ws.fixed() ? d->N > kAmpInKernelMaxN : amp_cast_first(d->M, d->N, d->K))) &&
         (!direct || ws.room(sizeof(_Float16) * (size_t)d->M * d->K)))
         return amp_via_cast(d, heads, nheads, head_cols, handoff, &ws);
     // scattered C needs the kernels with a plain or bias epilogue kind

@@ -3,11 +3,15 @@
 // gfx950's matrix cores multiply bf16 sixteen times as fast as binary32, and a
 // binary32 significand (24 bits) is exactly three bf16 significands (8 bits
 // each): x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 - x2
-// (round to nearest even, every difference exact).  A product then is
+// (round to nearest even, every difference exact; |x2| <= 2^-8 |x|, |x3| <=
+// 2^-17 |x|).  A product then is
 //     x y = x1 y1 + (x1 y2 + x2 y1) + (x1 y3 + x3 y1 + x2 y2) + r,
 // six bf16 products, each exact in the MFMA's binary32 accumulation, and
-// |r| <= |x2 y3| + |x3 y2| + |x3 y3| < 2^-25 |x y|: below the half ulp (2^-24)
-// of one binary32 rounding.  Six bf16 MFMAs cover 16 contraction steps in the
+// |r| <= |x2 y3| + |x3 y2| + |x3 y3| <= 2^-24 (1 + 2^-10) |x y|: as much as one
+// binary32 rounding at worst (x = y = 1 + 2^-8 - 2^-17 loses 0.99 of it), made
+// good by rounding sums once per 16 steps (Henry, Tang, Heinecke, "Leveraging
+// the bfloat16 artificial intelligence datatype for higher-precision
+// computations", ARITH 2019).  Six bf16 MFMAs cover 16 contraction steps in the
 // time v_mfma_f32_32x32x2_f32 covers 6: 2.67 times the binary32 rate.
 //
 // Measured against float64 (32 x 32 tiles, K contraction steps, relative
@@ -19,11 +23,11 @@
 // Range.  The bf16 MFMA flushes subnormal operands, so values are scaled by
 // 2^24 before the split: the last bit of any binary32 value, the smallest
 // subnormal (2^-149) included, then is at least 2^-125 and every part is zero
-// or normal.  Checked bit for bit over [2^-149, 2^104) (4 Mi values per range).
-// A value of 2^104 or more, an infinity or a NaN makes the parts, and so the
-// sums they enter, infinite or NaN; so does a scaled sum of 2^128 or more.  The
-// kernels check their sums for that and repeat such a block with
-// v_mfma_f32_32x32x2_f32 on the unscaled values.
+// or normal.  (The attention kernels distribute the factors as their sums
+// need them.)  A value that rounds to 2^104 or more in bf16, an infinity or a
+// NaN makes the parts, and so the sums they enter, infinite or NaN; so does a
+// scaled sum of 2^128 or more.  The kernels check their sums for that and repeat
+// such a block with v_mfma_f32_32x32x2_f32 on the unscaled values.
 #pragma once
 
 #include "vedic_common.hpp"

@@ -204,7 +204,8 @@ def amp_gemm(A: torch.Tensor, W16: torch.Tensor | None, W32: torch.Tensor | None
              preact: torch.Tensor | None = None) -> torch.Tensor:
     """The reference's amp_gemm / amp_gemm_bias (cuda/ModelGPU.cu:819-859) from a
     float32 activation A: C = binary16(A) . W16 (+ bias, then GELU if asked),
-    with A clamped and rounded to binary16 inside the GEMM (no cast pass); fp32
+    with A clamped and rounded to binary16 inside the GEMM or, for wide and long
+    products (see vedic_amp_gemm in logos_vedic.h), by a pass before it; fp32
     accumulation and output.  W16 None: the fp32 product with W32, the
     reference's fallback for a parameter without a binary16 shadow."""
     if A.dtype != torch.float32:
