@@ -280,7 +280,7 @@ __device__ __forceinline__ void fa_item(const FlashArgs& a, int item, int tid, c
 // once per item, P in registers.  Per block and wave DH / 16 x 6 MFMAs for S^T and
 // DH / 32 x 2 x 6 for O^T, 32 cycles each, against DH of 64 cycles on
 // v_mfma_f32_32x32x2_f32: 16 heads x seq 8192 causal 1218 -> 757 us, the
-// matrix pipe 62 % busy at 1.72 GHz, 6.4 VALU instructions (split, softmax) per
+// matrix pipe busy 59 % of the active cycles, 6.4 VALU instructions (split, softmax) per
 // MFMA beside it.  scale log2(e) goes into Q before the split, so the
 // scores come out in base 2.
 //

@@ -386,9 +386,8 @@ __device__ __forceinline__ void fb_dkdv_item(const FlashBwdArgs& a, int item, ch
 //
 // Bound: the matrix cores, 72 and 96 MFMAs of 32 cycles per 32 x 32 block
 // (fp32: 96 and 128 of 64).  16 heads x seq 8192 causal 4241 -> 2307 us per
-// backward (error against float64 2.2e-6 -> 1.6e-6): 61 and 60 % of the matrix
-// pipe busy at two waves per SIMD (246 and 254 registers), at the 1.83 GHz the
-// chip holds under this load.
+// backward (error against float64 2.2e-6 -> 1.6e-6), the matrix pipe busy 62 and
+// 59 % of the active cycles at two waves per SIMD (246 and 254 registers).
 // DH 128 (144 and 192 MFMAs per block): one wave per SIMD, 96 and 97 KB of LDS,
 // no spill; K, V, dK and dV of 32 keys fit beside two score blocks, so that S is
 // computed once for dK and dV.  8 heads x seq 8192 causal 5461 -> 2554 us per

@@ -357,8 +357,8 @@ gemm_f32s_kernel(GemmArgs args) {
 // Tile configurations.  Waves per SIMD (WPE) follow the registers: 128
 // accumulators per lane of the 256 x 256 tile leave two.  8192 x 8192 x 1024 NN
 // 595 us with 256 x 256 tiles (231 TFLOP/s; 1005 us on v_mfma_f32_32x32x2_f32),
-// 647 with 128 x 128: half the LDS reads and splits per MFMA, at 1.6 GHz (the
-// clock the chip holds under this load) 74 % of the matrix pipe busy.  One
+// 647 with 128 x 128: half the LDS reads and splits per MFMA, the matrix pipe
+// busy 69 % of the active cycles.  One
 // workgroup of 128 x 128 per CU reaches 177 TFLOP/s (4096 x 1024 x 8192).
 struct CfgSLarge {  // 256 x 256, eight waves of 128 x 64, one workgroup per CU
     static constexpr int BM = 256, BN = 256, WGM = 2, WGN = 4, WPE = 2, SETS = 1;
