@@ -983,8 +983,8 @@ hipError_t launch_gemm_f16_direct_op(const GemmArgs& a, hipStream_t s) {
     }
     if constexpr (OP == 3) {
         // fp32 A: no 256 x 256 or 256 x 192 tiles (its staging registers do
-        // not fit beside their accumulators); 256 x 128 where the cost model picks one of those three,
-        // else 128 x 128
+        // not fit beside their accumulators); 256 x 128 where the cost model
+        // picks one of those three, else 128 x 128
         if (a.ksplit <= 1 && f16_tile_config(a.M, a.N, device_cu_count()) != 2)
             return launch_f16_kind<OP, CfgMid>(a, s);
         return launch_f16_kind<OP, CfgSmall>(a, s);
