@@ -379,10 +379,15 @@ __device__ __forceinline__ void fb_dkdv_item(const FlashBwdArgs& a, int item, ch
 // Both passes with every operand split exactly into three bf16 parts
 // (vedic_split.hpp): the streamed blocks once per workgroup on their way into
 // LDS (two buffers, one barrier per 32 rows), the resident rows once per item,
-// P and dS in registers.  Every operand carries the split's factor 2^24, scale
-// log2(e) with the resident side of the score product: scores come out in base
-// 2 times 2^48, which the exponent takes out in its subtraction (an fma).  dP, D
-// and dS carry 2^48, the accumulators 2^72 (dV: 2^48).
+// P and dS in registers.  Every operand carries the split's factor 2^24, Q of the
+// score products scale log2(e) too: scores come out in base 2 times 2^48, which
+// the exponent takes out in its subtraction (an fma).  dP, D and dS carry 2^48,
+// dQ 2^72, dV 2^48, and dK 2^48 and Q's factor.
+// Both passes compute the forward's scores bit for bit (the factor on Q, the six
+// products in one order): their rounding is in lse too and cancels in P.  With
+// the factor on K in the dK/dV pass it did not, and dV and dK were further from
+// float64 the larger the scores (Q of N(0, 16^2), 300 rows, DH 64: dV 5.6e-6, dK
+// 6.5e-6; now 1.7e-6 and 3.1e-6; on the fp32 MFMA 2.3e-6 and 3.6e-6).
 //
 // Bound: the matrix cores, 72 and 96 MFMAs of 32 cycles per 32 x 32 block
 // (fp32: 96 and 128 of 64).  16 heads x seq 8192 causal 4241 -> 2307 us per
@@ -545,7 +550,8 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
     const bool live = k0 < a.seq;
 
     SplitFrag kf[DH / 16], vf[DH / 16];
-    fs_load_rows<DH>(kf, a.k[head], key, a.seq, a.scale * (1.4426950408889634f * kSplitScale), lane);
+    const float qscale = a.scale * (1.4426950408889634f * kSplitScale);
+    fs_load_rows<DH>(kf, a.k[head], key, a.seq, kSplitScale, lane);
     fs_load_rows<DH>(vf, a.v[head], key, a.seq, kSplitScale, lane);
     const float* stats = a.delta + (int64_t)head * a.seq * 2;
 
@@ -568,7 +574,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
         st = in ? (tid & 1 ? st * kFbScale2 : st) : tid & 1 ? 0.0f : __builtin_inff();
     };
     auto commit = [&](char* buf) {
-        sq.commit(buf, kSplitScale, tid);
+        sq.commit(buf, qscale, tid);
         sd.commit(buf + KB, kSplitScale, tid);
         if (tid < 64) *reinterpret_cast<float*>(buf + 2 * KB + (tid & 1) * 128 + (tid >> 1) * 4) = st;
     };
@@ -576,7 +582,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
         const char* sl = buf + 2 * KB + 16 * h;
         float16_t s = float16_t{};
 #pragma unroll
-        for (int j = 0; j < DH / 16; ++j) s = mfma_split(fs_row<DH>(buf, ad, j), kf[j], s);
+        for (int j = 0; j < DH / 16; ++j) s = mfma_split_swapped(fs_row<DH>(buf, ad, j), kf[j], s);
         // s[4 gg + r]: query qb0 + 8 gg + 4 h + r against this lane's key
 #pragma unroll
         for (int i = 0; i < 16; ++i) low = fminf(low, s[i]);
@@ -643,6 +649,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
     // (keys past seq are not stored: their sums may be anything)
     if (__syncthreads_or(key < a.seq && (probe != 0.0f || low == -__builtin_inff()))) return false;
     if (!live || key >= a.seq) return true;
+    const float kscale = qscale != 0.0f ? a.scale / qscale : 0.0f;
     float* vrow = a.dv[head] + (int64_t)key * DH;
     float* krow = a.dk[head] + (int64_t)key * DH;
 #pragma unroll
@@ -653,7 +660,7 @@ __device__ __forceinline__ bool fb_dkdv_split(const FlashBwdArgs& a, int item, c
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 v[r] = dv[d][4 * gg + r] * kSplitUnscale2;
-                w[r] = dk[d][4 * gg + r] * kFbUnscale3 * a.scale;
+                w[r] = dk[d][4 * gg + r] * kSplitUnscale2 * kscale;
             }
             store16_hold(vrow + 32 * d + 8 * gg + 4 * h, v);
             store16_hold(krow + 32 * d + 8 * gg + 4 * h, w);

@@ -64,10 +64,7 @@ struct FsStage {
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             const int u = i * NT + tid, row = u / CPR, c = u % CPR;
-            float w[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) w[e] = scale == 1.0f ? v[i][e] : v[i][e] * scale;
-            const SplitFrag f = split8(w);
+            const SplitFrag f = split8(v[i], scale);
             char* dst = lds + row * 6 * DH + ((c ^ fs_swz<DH>(row)) << 4);
 #pragma unroll
             for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8_t*>(dst + p * 2 * DH) = f.p[p];
@@ -139,9 +136,9 @@ __device__ __forceinline__ void fs_load_rows(SplitFrag (&f)[DH / 16], const floa
             const float4_t t = __builtin_bit_cast(
                 float4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off == kOob ? kOob : off + 64 * j + 16 * q), 0, 0));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) w[4 * q + e] = t[e] * scale;
+            for (int e = 0; e < 4; ++e) w[4 * q + e] = t[e];
         }
-        f[j] = split8(w);
+        f[j] = split8(w, scale);
     }
 }
 
@@ -150,8 +147,8 @@ __device__ __forceinline__ void fs_load_rows(SplitFrag (&f)[DH / 16], const floa
 __device__ __forceinline__ SplitFrag fs_acc(const float16_t& s, int j, float scale) {
     float w[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) w[e] = scale == 1.0f ? s[8 * j + e] : s[8 * j + e] * scale;
-    return split8(w);
+    for (int e = 0; e < 8; ++e) w[e] = s[8 * j + e];
+    return split8(w, scale);
 }
 
 }  // namespace vedic

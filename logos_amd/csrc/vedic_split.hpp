@@ -69,12 +69,42 @@ struct SplitFrag {
     bf16x8_t p[3];
 };
 
+// The same of scale x and scale y: the first remainder is taken from the exact
+// product, spelled out so that every kernel splits a value alike (the compiler
+// would contract the multiplication into the subtraction in some and not in
+// others, and scores that two kernels compute for one probability would differ).
+__device__ __forceinline__ SplitPair split_pair(float x, float y, float scale) {
+    SplitPair s;
+    s.p[0] = __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t{x * scale, y * scale}), bf16x2_t));
+    x = __builtin_fmaf(x, scale, -__builtin_bit_cast(float, s.p[0] << 16));
+    y = __builtin_fmaf(y, scale, -__builtin_bit_cast(float, s.p[0] & 0xFFFF0000u));
+    s.p[1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t{x, y}), bf16x2_t));
+    x -= __builtin_bit_cast(float, s.p[1] << 16);
+    y -= __builtin_bit_cast(float, s.p[1] & 0xFFFF0000u);
+    s.p[2] = __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t{x, y}), bf16x2_t));
+    return s;
+}
+
 // Eight values -> their parts.
 __device__ __forceinline__ SplitFrag split8(const float (&v)[8]) {
     u32x4_t w[3];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const SplitPair s = split_pair(v[2 * e], v[2 * e + 1]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) w[p][e] = s.p[p];
+    }
+    SplitFrag f;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) f.p[p] = __builtin_bit_cast(bf16x8_t, w[p]);
+    return f;
+}
+
+__device__ __forceinline__ SplitFrag split8(const float (&v)[8], float scale) {
+    u32x4_t w[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const SplitPair s = split_pair(v[2 * e], v[2 * e + 1], scale);
 #pragma unroll
         for (int p = 0; p < 3; ++p) w[p][e] = s.p[p];
     }
@@ -95,6 +125,14 @@ __device__ __forceinline__ float16_t mfma_split(const SplitFrag& a, const SplitF
 #pragma unroll
     for (int q = 0; q < kSplitProducts; ++q)
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[kSplitA[q]], b.p[kSplitB[q]], acc, 0, 0, 0);
+    return acc;
+}
+
+// The same with the roles of a and b exchanged: b . a has these bits.
+__device__ __forceinline__ float16_t mfma_split_swapped(const SplitFrag& a, const SplitFrag& b, float16_t acc) {
+#pragma unroll
+    for (int q = 0; q < kSplitProducts; ++q)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[kSplitB[q]], b.p[kSplitA[q]], acc, 0, 0, 0);
     return acc;
 }
 

@@ -237,6 +237,34 @@ def test_backward_tiny_probabilities(dh, t):
     assert np.abs(got - want).max() <= (4 * t + 4 * np.sqrt(seq)) * o.U32 * size
 
 
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("std", [1.0, 6.0])
+def test_passes_recompute_the_same_probabilities(dh, std):
+    """P of one key, read out of each backward pass bit for bit: of the dK/dV pass
+    by unit rows of dO (dV[key] = P), of the dQ pass by a unit value of V and O =
+    0 (dS = P on that key, whose K has a 1).  A rounding of the scores that the
+    two passes, and the forward that made lse, share cancels; one that differs
+    is an error of P of its size."""
+    v = vedic()
+    rng = np.random.default_rng(41 + dh)
+    seq, key, scale = 150, 37, 0.125
+    Q, K = normal(rng, (seq, dh)) * np.float32(std), normal(rng, (seq, dh))
+    K[:, dh - 1] = 0
+    K[key, dh - 1] = 1
+    lse = torch.empty(seq, device="cuda")
+    v.flash_attention_fwd(dev(Q), dev(K), dev(K), lse=lse, scale=scale, causal=False)
+    zero = np.zeros((seq, dh), np.float32)
+    one, V = zero.copy(), zero.copy()
+    one[np.arange(dh), np.arange(dh)] = 1.0  # dO of the first dh queries
+    dV = host(v.flash_attention_bwd(dev(Q), dev(K), dev(zero), dev(zero), dev(one), lse, scale=scale, causal=False)[2])
+    V[key, 0] = 1.0
+    dO = zero.copy()
+    dO[:, 0] = 1.0
+    dQ = host(v.flash_attention_bwd(dev(Q), dev(K), dev(V), dev(zero), dev(dO), lse, scale=scale, causal=False)[0])
+    assert np.all(dV[key, :] > 0)
+    assert np.array_equal(dV[key, :], dQ[:dh, dh - 1] / np.float32(scale))
+
+
 def test_backward_nonfinite():
     """A NaN in one dO row reaches every dK, dV row it attends to and its own
     dQ row; the other queries keep their finite dQ and the keys past its
