@@ -222,8 +222,13 @@ struct Workspace {
     bool capturing() {
         if (captured < 0) {
             hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-            captured = s != nullptr && hipStreamGetCaptureInfo(s, &st, &capture_id) == hipSuccess &&
-                       st != hipStreamCaptureStatusNone;
+            captured = 0;
+            if (s != nullptr) {
+                if (hipStreamGetCaptureInfo(s, &st, &capture_id) != hipSuccess)
+                    (void)hipGetLastError();  // (not the error of this call's launches)
+                else
+                    captured = st != hipStreamCaptureStatusNone;
+            }
         }
         return captured != 0;
     }
